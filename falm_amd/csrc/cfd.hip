@@ -205,6 +205,7 @@ constexpr int KM_HPT = (KM_HALO + KM_NT - 1) / KM_NT;  // halo cells per thread
 struct KmTiling {
     Box box;
     int tx, ty, tk;  // column tiles along x, y and k chunks
+    int kc;          // planes per chunk (at most KM_KC)
     int blocks;
 };
 inline KmTiling make_km_tiling(const Box &b) {
@@ -212,7 +213,8 @@ inline KmTiling make_km_tiling(const Box &b) {
     t.box = b;
     t.tx = (b.n[0] + KM_BX - 1) / KM_BX;
     t.ty = (b.n[1] + KM_BY - 1) / KM_BY;
-    t.tk = (b.n[2] + KM_KC - 1) / KM_KC;
+    t.kc = k7_chunk(t.tx * t.ty, b.n[2], KM_KC);
+    t.tk = (b.n[2] + t.kc - 1) / t.kc;
     t.blocks = t.tx * t.ty * t.tk;
     return t;
 }
@@ -259,8 +261,8 @@ __global__ __launch_bounds__(KM_NT) void k_pseudo_u_km(KmTiling kt, Geom g, T Re
     const int i0 = kt.box.lo[0] + bx * KM_BX, j0 = kt.box.lo[1] + by * KM_BY;
     const int i = i0 + lane, j = j0 + wy;
     const bool act = i < kt.box.lo[0] + kt.box.n[0] && j < kt.box.lo[1] + kt.box.n[1];
-    const int k0 = kt.box.lo[2] + kc * KM_KC;
-    const int k1 = min(k0 + KM_KC, kt.box.lo[2] + kt.box.n[2]);
+    const int k0 = kt.box.lo[2] + kc * kt.kc;
+    const int k1 = min(k0 + kt.kc, kt.box.lo[2] + kt.box.n[2]);
     const int sy = g.nx, sz = g.nxy;
     // Threads past the box still load their own cell into the LDS plane
     // when it lies in the array: the last active columns and rows read it
@@ -474,8 +476,8 @@ __global__ __launch_bounds__(KM_NT) void k_pseudo_u3_km(KmTiling kt, Geom g, T R
     const int i0 = kt.box.lo[0] + bx * KM_BX, j0 = kt.box.lo[1] + by * KM_BY;
     const int i = i0 + lane, j = j0 + wy;
     const bool act = i < kt.box.lo[0] + kt.box.n[0] && j < kt.box.lo[1] + kt.box.n[1];
-    const int k0 = kt.box.lo[2] + kc * KM_KC;
-    const int k1 = min(k0 + KM_KC, kt.box.lo[2] + kt.box.n[2]);
+    const int k0 = kt.box.lo[2] + kc * kt.kc;
+    const int k1 = min(k0 + kt.kc, kt.box.lo[2] + kt.box.n[2]);
     const int sy = g.nx, sz = g.nxy;
     const unsigned syb = (unsigned)sy * TS, szb = (unsigned)sz * TS;
     // as in k_pseudo_u_km: threads past the box load their own cell when it

@@ -27,17 +27,38 @@ struct K7Tiling {
     int blocks;
 };
 
-// planes per chunk: K7_KC, doubled until the grid fits max_blocks workgroups
+// Planes per chunk of the k-marching kernels: K7_KC, doubled until the grid
+// fits max_blocks workgroups, and shortened while the grid has fewer than
+// K7_FILL.  A workgroup walks its planes one after the other (0.5 us a plane
+// and more), so a small domain's time is its chunk length and not its bytes:
+// 64 x 33 x 30 cells are 5 columns, with 16-plane chunks 10 workgroups on 256
+// CUs (pseudo-velocity 30 us, 17 us Smagorinsky and divergence).  The line
+// lies at two workgroups a CU: on MI355X the wind-tunnel step in double took
+// 660 us at 64 x 33 x 30 with 16 planes a chunk, 416 us filled to 256
+// workgroups and 400 us to 512; at 128^3 cells two k_sor3_km workgroups fit a
+// CU (LDS), and the cavity solve took 1109 us unfilled, 960 us at 512 and
+// 1075 us at 1024.
 #ifndef FALM_K7_KC
 #define FALM_K7_KC 16
 #endif
 constexpr int K7_KC = FALM_K7_KC;
+constexpr int K7_FILL = 512;
+
+// chunk length (at most kc planes of nz) at which cols columns of chunks
+// make about K7_FILL workgroups
+inline int k7_chunk(int cols, int nz, int kc) {
+    if (cols < 1) cols = 1;
+    const int tk = (K7_FILL + cols - 1) / cols;  // chunks per column wanted
+    const int k = (nz + tk - 1) / tk;
+    return k < 1 ? 1 : k < kc ? k : kc;
+}
+
 inline K7Tiling make_k7_tiling(const Box &b, int max_blocks = RED_BLOCKS) {
     K7Tiling t;
     t.box = b;
     t.tx = (b.n[0] + K7_BX - 1) / K7_BX;
     t.ty = (b.n[1] + K7_BY - 1) / K7_BY;
-    t.kc = K7_KC;
+    t.kc = k7_chunk(t.tx * t.ty, b.n[2], K7_KC);
     for (;;) {
         t.tk = (b.n[2] + t.kc - 1) / t.kc;
         t.blocks = t.tx * t.ty * t.tk;
@@ -48,7 +69,7 @@ inline K7Tiling make_k7_tiling(const Box &b, int max_blocks = RED_BLOCKS) {
     return t;
 }
 
-// the shortest chunk (at least K7_KC planes) whose grid fits max_blocks
+// the shortest chunk whose grid fits max_blocks
 inline K7Tiling make_k7_tiling_fit(const Box &b, int max_blocks) {
     K7Tiling t;
     t.box = b;
@@ -58,7 +79,7 @@ inline K7Tiling make_k7_tiling_fit(const Box &b, int max_blocks) {
     int tk = max_blocks / cols;
     if (tk < 1) tk = 1;
     t.kc = (b.n[2] + tk - 1) / tk;
-    if (t.kc < K7_KC) t.kc = K7_KC;
+    if (t.kc < 1) t.kc = 1;
     t.tk = (b.n[2] + t.kc - 1) / t.kc;
     t.blocks = t.tx * t.ty * t.tk;
     if (b.n[0] <= 0 || b.n[1] <= 0 || b.n[2] <= 0) t.blocks = 0;

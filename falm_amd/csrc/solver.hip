@@ -426,11 +426,15 @@ static_assert((PQ_R1T0 + 2 * K7_BY) % 64 == 0, "ring-1 rows start on a wave");
 template <class T>
 using PQLds = T[4][PQ_H][PQ_W];
 // k_bicg_pcmv_km runs one round of workgroups, pcmv_wg_per_cu of them
-// resident on each CU: its chunk is the shortest (at least K7_KC planes)
-// whose grid fits that many.  Float kernels run two 8-wave workgroups per CU
+// resident on each CU: its chunk is the shortest whose grid fits that many.
+// Float kernels run two 8-wave workgroups per CU
 // (at most 128 VGPRs, which the separable-operator instances are held to);
 // double ones one, with 64-plane chunks at 512 x 128 x 128 (measured as fast
 // as two per CU, and the folded double s kernel needs more than 128 VGPRs).
+// Small domains get short chunks: a step (0.5 us and more) costs a workgroup
+// the same whatever the grid, and a chunk of n planes takes n + 4 of them.
+// With chunks of at least 16 planes a double iteration took 56 us at
+// 96 x 48 x 48 (36 workgroups); at 3 planes (192) it takes 23 us.
 #ifndef FALM_PCMV_WG_F32
 #define FALM_PCMV_WG_F32 2
 #endif
@@ -797,13 +801,14 @@ constexpr int S3_RB = 2;                    // b / diagonal ring
 constexpr int S3_BW = S3_BX + 2 * S3_RB, S3_BH = S3_BY + 2 * S3_RB;
 constexpr int S3_BPL = S3_BW * S3_BH;       // b cells per plane
 constexpr int S3_NBP = 3;                   // b planes in flight: s+1 .. s-1
-constexpr int S3_KC = 16;                   // output planes per chunk
+constexpr int S3_KC = 16;                   // output planes per chunk at most
 constexpr int S3_XPT = (S3_PL + S3_NT - 1) / S3_NT;   // x cells per thread per plane
 constexpr int S3_BPT = (S3_BPL + S3_NT - 1) / S3_NT;  // b cells per thread per plane
 
 struct S3Tiling {
     Box box;  // the interior
     int tx, ty, tk;
+    int kc;  // output planes per chunk
     int blocks;
 };
 inline S3Tiling make_s3_tiling(const Box &b) {
@@ -811,7 +816,8 @@ inline S3Tiling make_s3_tiling(const Box &b) {
     t.box = b;
     t.tx = (b.n[0] + S3_BX - 1) / S3_BX;
     t.ty = (b.n[1] + S3_BY - 1) / S3_BY;
-    t.tk = (b.n[2] + S3_KC - 1) / S3_KC;
+    t.kc = k7_chunk(t.tx * t.ty, b.n[2], S3_KC);
+    t.tk = (b.n[2] + t.kc - 1) / t.kc;
     t.blocks = (b.n[0] > 0 && b.n[1] > 0 && b.n[2] > 0) ? t.tx * t.ty * t.tk : 0;
     return t;
 }
@@ -830,7 +836,7 @@ __global__ __launch_bounds__(S3_NT) void k_sor3_km(S3Tiling kt, Geom g, OpSep<T>
     const int ilo = kt.box.lo[0], ihi = kt.box.lo[0] + kt.box.n[0];  // interior [lo, hi)
     const int jlo = kt.box.lo[1], jhi = kt.box.lo[1] + kt.box.n[1];
     const int klo = kt.box.lo[2], khi = kt.box.lo[2] + kt.box.n[2];
-    const int k0 = klo + kc * S3_KC, k1 = min(k0 + S3_KC, khi);  // output planes
+    const int k0 = klo + kc * kt.kc, k1 = min(k0 + kt.kc, khi);  // output planes
     const int t = (int)threadIdx.x;
     const int sz = g.nxy;
     // 1-D operator coefficients of the tile's x and y range
