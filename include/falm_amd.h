@@ -456,8 +456,11 @@ falm_status falm_case_adjoint_attitude(falm_case *c, double *g_yaw, double *g_of
  * stages above, the transposes the rotor-power adjoint chains: given the
  * adjoint of a stage's output, each adds the adjoint of its inputs to the
  * *bar outputs (+=, so several contributions accumulate), except where
- * noted.  FP64 device arrays in the Matrix layout; atomics make the sums
- * order-independent to rounding (not bitwise reproducible from run to run).
+ * noted.  FP64 device arrays in the Matrix layout.  Whole-field stages add to
+ * each output cell once, in a fixed order; the boundary fills and
+ * falm_alm_vjp use atomics (order-independent to rounding, not bitwise
+ * reproducible from run to run).  Calls that accumulate into the same output
+ * must be ordered on one stream.
  * The *bar outputs (and falm_alm_vjp's g_pitch, g_twist) must be device
  * memory from hipMalloc: the kernels accumulate into them with hardware FP64
  * atomic adds, which can drop updates on host-pinned, managed or

@@ -1,8 +1,8 @@
 """Per-stage adjoints (VJPs) of the HIP library through the C ABI.
 
 Each is checked two ways: against the oracle's transpose of the same stage
-on seeded inputs (1e-12 relative; the device gathers or adds with atomics,
-so only the order of additions differs), and, independently of the oracle,
+on seeded inputs (1e-12 relative; the device gathers, or at the boundary and
+the rotor adds with atomics, so only the order of additions differs), and, independently of the oracle,
 against the library's own forward stage on the GPU: the transposition identity
 <J v, w> = <v, J^T w> for the linear stages and central differences for the
 nonlinear ones (pseudo-velocity, Smagorinsky, actuator line)."""
@@ -173,6 +173,38 @@ def test_pseudo_u_vjp(gpu, scheme):
     fd = (ua_at(eps) - ua_at(-eps)) @ w / (2 * eps)
     ad = vu @ g_u + vuu @ g_uu + vnut @ g_nut + vff @ g_ff
     assert abs(fd - ad) <= 1e-6 * abs(fd)
+
+
+# one cell; thin boxes; the Smagorinsky tile's last output column and row
+# (60 + 2 = 62, 4 + 2 = 6) and one beyond; several chunks of planes
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 3, 1), (60, 4, 5), (61, 5, 3), (130, 13, 40)])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_gathered_vjps_at_edges(gpu, n, sparse):
+    """The gathered pseudo-velocity and Smagorinsky transposes where their
+    stencils leave the interior on both sides and where tiles end, added to
+    outputs that already hold something; sparse: an adjoint that is zero at
+    most cells.  Each sum has at most ~200 terms: 1e-12 of the largest."""
+    dom = domain(n)
+    rng, F = _fields(dom, 77)
+    ReI, dt, Cs = 1.0 / 2500.0, 2e-3, 0.12
+    w = rng.standard_normal(3 * dom.ncell) * interior_mask(dom, 3)
+    wn = rng.standard_normal(dom.ncell) * interior_mask(dom)
+    if sparse:
+        w *= rng.random(w.size) < 0.05
+        wn *= rng.random(wn.size) < 0.05
+    d = {k: to_dev(v) for k, v in F.items()}
+    wd, wnd = to_dev(w), to_dev(wn)
+    had = [rng.standard_normal(m * dom.ncell) for m in (3, 3, 1, 3)]
+    out = [to_dev(v) for v in had]
+    gpu.call("falm_pseudo_u_vjp", C.byref(dom), abi.ADV_UPWIND3, ReI, dt,
+             *_ptrs(gpu, d["u"], d["uu"], d["nut"], d["kx"], d["g"], d["ja"], wd, *out), None)
+    ref = O.adj_pseudo_u(dom, 1 / 24, ReI, dt, F["u"], F["uu"], F["nut"], F["kx"], F["g"], F["ja"], w)
+    for q, (a, b, h) in enumerate(zip(out, ref, had)):
+        b = np.where(interior_mask(dom, 3), b, h) if q == 3 else b + h  # ffbar is overwritten on the interior
+        assert rel_err(from_dev(a), b) < TOL, q
+    ub = to_dev(had[0])
+    gpu.call("falm_sgs_vjp", C.byref(dom), Cs, *_ptrs(gpu, d["u"], d["kx"], d["ja"], wnd, ub), None)
+    assert rel_err(from_dev(ub), O.adj_sgs(dom, Cs, F["u"], F["kx"], F["ja"], wn) + had[0]) < TOL
 
 
 def test_pseudo_u_vjp_rejects_other_schemes(gpu):
