@@ -1446,6 +1446,253 @@ __global__ __launch_bounds__(FIN_NT) void k_fin_resnorm(DevState *st, const doub
     }
 }
 
+// ---------------------------------------------------------------------
+// The SOR solver (src/FalmEq.cpp:173-240) on a domain of one interior layer:
+// K iterations (black half-sweep, red half-sweep, |b - A x|^2) in one launch.
+// Such domains are small (the 2-D cavity's 128 x 128 cells are 2 us of traffic
+// for one XCD), so an iteration of four launches (two half-sweeps, residual,
+// finalize) is launch time: 12.6 us.  A workgroup owns a TX x TY tile and
+// iterates on the tile and a ring of R = 2 K + 1 cells in LDS, redundantly:
+// every half-sweep makes one more ring layer stale, and after K iterations
+// the tile and the one layer its residual reads are still exact, so the
+// iterates are those of separate sweeps, up to rounding.  Each thread owns one
+// black and one red cell of the region with their coefficients in registers;
+// the two colours lie in LDS arrays of their own, so that the lanes of a
+// half-sweep are adjacent.  A red cell's residual reads what its update read,
+// a black cell's is the b - A x of the next black half-sweep: an iteration is
+// two barriers.
+//
+// x is double-buffered over launches (launch L reads x, the solver's own
+// vector xw in turn).  The stop test of an iteration is made by the next
+// launch, in which every workgroup sums the K norms' partials in the same
+// order.  If the solve ended inside the previous launch, that launch's input
+// is still there, and this one repeats the iterations that count; if it ended
+// with it, nothing is left to do.  The workgroups of one launch must agree
+// though one of them sets `done`: it holds the launch's number + 1, and only
+// later launches return on it.  k_sor2d_out then brings x (and the residual)
+// home.
+//
+// Measured at 128 x 128: a launch takes 7 us (3 of them that of an empty one;
+// the rest loads, the norms' sums) and 0.6 to 1 us an iteration: 10 us at
+// K = 4, 11.2 at 6, 12.2 at 7.  More iterations need a wider ring, so the
+// smallest domains take the most: the line lies where each workgroup sums all
+// partials and every workgroup finds a CU of its own.
+template <int K_, int TX_, int TY_, int MAXWG_>
+struct S2Cfg {
+    static constexpr int K = K_, TX = TX_, TY = TY_, MAXWG = MAXWG_, NT = 1024;
+    static constexpr int R = 2 * K + 1;
+    static constexpr int HW = (TX + 2 * R) / 2, H = TY + 2 * R;  // cells of a colour in a row, rows
+    static constexpr int NC = HW * H;
+    static_assert(NC <= NT && TX % 2 == 0, "one cell of a colour per thread");
+    static_assert(K * MAXWG <= NT && MAXWG % 64 == 0, "one partial per thread, whole waves per norm");
+};
+using S2A = S2Cfg<7, 12, 12, 128>;   // up to 128 x 144 cells, say
+using S2B = S2Cfg<6, 16, 16, 128>;   // up to 176 x 176
+using S2C = S2Cfg<4, 32, 16, 256>;   // up to 512 x 256; larger ones run separate sweeps
+
+struct S2Tiling {
+    Box box;
+    int tx, ty, blocks, cfg;  // no blocks: the general path
+};
+template <class C>
+inline bool s2_fits(const Box &b, S2Tiling &t, int cfg) {
+    t.tx = (b.n[0] + C::TX - 1) / C::TX;
+    t.ty = (b.n[1] + C::TY - 1) / C::TY;
+    t.cfg = cfg;
+    const long long nb = (long long)t.tx * t.ty;
+    t.blocks = nb <= C::MAXWG ? (int)nb : 0;
+    return t.blocks > 0;
+}
+inline S2Tiling make_s2_tiling(const Box &b) {
+    S2Tiling t{b, 0, 0, 0, 0};
+    if (b.n[0] > 0 && b.n[1] > 0 && b.n[2] == 1 && !s2_fits<S2A>(b, t, 0) && !s2_fits<S2B>(b, t, 1))
+        s2_fits<S2C>(b, t, 2);
+    return t;
+}
+inline int s2_k(const S2Tiling &t) { return t.cfg == 0 ? S2A::K : t.cfg == 1 ? S2B::K : S2C::K; }
+
+// One cell of the region: its coefficients, x, and b without the two z
+// neighbours' products, which do not change.  The residual is summed as a
+// tree and the division is a product with the stored reciprocal corrected by
+// one fused step (correctly rounded but for ties of two ulps): a half-sweep is
+// one chain of dependent double operations, 7 this way, 28 as a running sum
+// and a division.
+struct S2Cell {
+    double ac, aw, ae, as, an, b, x, ra;
+    int cc;
+    bool inner, upd, out;  // an interior cell; updated here; in the tile (stored and counted)
+    __device__ inline double res(double xe, double xw, double xn, double xs) const {
+        return fma(-ac, x, b) - (fma(aw, xw, ae * xe) + fma(as, xs, an * xn));
+    }
+    __device__ inline double over_ac(double v) const {
+        const double q = v * ra;
+        return fma(fma(-ac, q, v), ra, q);
+    }
+};
+
+template <class OP, class C>
+__global__ __launch_bounds__(C::NT) void k_sor2d(S2Tiling tl, Geom g, OP a, double *x, double *xw,
+                                                 const double *__restrict__ b, double omega, DevState *st,
+                                                 const double *__restrict__ pin, double *__restrict__ pout, int L) {
+    constexpr int S2_K = C::K, S2_TX = C::TX, S2_TY = C::TY, S2_NT = C::NT, S2_R = C::R, S2_HW = C::HW, S2_H = C::H,
+                  S2_NC = C::NC;
+    const int dn = st->done;
+    __shared__ double lx[2][S2_NC];  // black, red
+    __shared__ double red[S2_K][S2_NT / 64];
+    const int tid = (int)threadIdx.x, nwg = (int)gridDim.x;
+    const int lane = tid & 63, wid = tid >> 6;
+    const double *src = (L & 1) ? xw : x;
+    double *dst = (L & 1) ? x : xw;
+    // this thread's black and red cell
+    const int bx = (int)blockIdx.x % tl.tx, by = (int)blockIdx.x / tl.tx;
+    const int gc = g.gc, k = tl.box.lo[2];
+    const int i0 = tl.box.lo[0] + bx * S2_TX - S2_R, j0 = tl.box.lo[1] + by * S2_TY - S2_R;
+    const int ry = tid / S2_HW, px = tid - ry * S2_HW;
+    const bool own = tid < S2_NC;
+    // x offset of the row's black cells: (i + j + k + osum) even
+    const int o = (i0 + j0 + ry + k + g.osum) & 1;
+    // both cells' operands are loaded before either is used (at an interior
+    // cell where the region leaves the array)
+    struct Raw {
+        double ac, aw, ae, as, an, ab, at, b, x, xt, xb;
+    };
+    const auto place = [&](int rx, S2Cell &c, Raw &q) {
+        int i = i0 + rx, j = j0 + ry;
+        const bool in = own && i >= 0 && i < g.nx && j >= 0 && j < g.ny;
+        i = in ? i : gc;
+        j = in ? j : gc;
+        c.inner = in && i >= gc && i < g.nx - gc && j >= gc && j < g.ny - gc;
+        c.upd = c.inner && rx >= 1 && rx < 2 * S2_HW - 1 && ry >= 1 && ry < S2_H - 1;
+        c.out = c.inner && rx >= S2_R && rx < S2_R + S2_TX && ry >= S2_R && ry < S2_R + S2_TY;
+        c.cc = g.id(i, j, k);
+        q.x = c.inner ? src[c.cc] : x[c.cc];
+        a.get(c.cc, i, j, k, q.ac, q.aw, q.ae, q.as, q.an, q.ab, q.at);
+        q.b = b[c.cc];
+        q.xt = x[c.cc + g.nxy];
+        q.xb = x[c.cc - g.nxy];
+    };
+    const auto make = [](S2Cell &c, const Raw &q) {
+        c.ac = q.ac;
+        c.aw = q.aw;
+        c.ae = q.ae;
+        c.as = q.as;
+        c.an = q.an;
+        c.x = q.x;
+        c.b = fma(-q.ab, q.xb, fma(-q.at, q.xt, q.b));
+        c.ra = 1.0 / q.ac;
+    };
+    S2Cell cb, cr;
+    Raw qb, qr;
+    place(2 * px + o, cb, qb);
+    place(2 * px + 1 - o, cr, qr);
+    if (dn && dn != L + 1) return;
+    int mrun = S2_K;
+    if (L > 0) {
+        // (the cells' operands are in flight meanwhile)
+        // the norms of the previous launch's iterations: G threads each
+        constexpr int G = C::MAXWG;
+        const int q = tid / G, w0 = tid % G;
+        double v = w0 < nwg && q < S2_K ? pin[q * nwg + w0] : 0.0;
+        v = wave_sum(v);
+        if (lane == 0) red[0][wid] = v;
+        __syncthreads();
+        int stop = 0;
+        double err = 0.0;
+        const int base = (L - 1) * S2_K;
+#pragma unroll
+        for (int m = 0; m < S2_K; m++) {
+            double t = 0.0;
+#pragma unroll
+            for (int w = 0; w < G / 64; w++) t += red[0][m * (G / 64) + w];
+            const double e = sqrt(t) / st->gN;
+            if (!stop && !(base + m + 1 < st->maxit && e > st->tol)) {
+                stop = m + 1;
+                err = e;
+            }
+        }
+        __syncthreads();  // red is reused below
+        if (stop) {  // uniform
+            if (blockIdx.x == 0 && tid == 0) {
+                st->it_pass = base + stop;
+                st->err = err;
+                st->plast = L & 1;  // the previous launch's output (1: xw)
+                st->done = L + 1;
+            }
+            if (stop == S2_K) return;
+            mrun = stop;  // repeat them from the previous launch's input
+            if (cb.inner) qb.x = dst[cb.cc];
+            if (cr.inner) qr.x = dst[cr.cc];
+            dst = (L & 1) ? xw : x;
+        }
+    }
+    make(cb, qb);
+    make(cr, qr);
+    if (own) {
+        lx[0][tid] = cb.x;
+        lx[1][tid] = cr.x;
+    }
+    __syncthreads();
+    double acc[S2_K];
+#pragma unroll
+    for (int m = 0; m < S2_K; m++) acc[m] = 0.0;
+    // neighbours in the other colour's array: west, east, south, north
+    const int wb = tid + o - 1, wr = tid - o, sn = tid - S2_HW, nn = tid + S2_HW;
+#pragma unroll
+    for (int m = 0; m <= S2_K; m++) {
+        if (m > mrun) break;
+        if (cb.upd) {  // black: the residual of iteration m - 1, then the update of iteration m
+            const double rv = cb.res(lx[1][wb + 1], lx[1][wb], lx[1][nn], lx[1][sn]);
+            if (m > 0 && cb.out) acc[m - 1] += rv * rv;
+            if (m < mrun) {
+                cb.x = cb.x + omega * cb.over_ac(rv);
+                lx[0][tid] = cb.x;
+            }
+        }
+        if (m == mrun) break;
+        __syncthreads();
+        if (cr.upd) {
+            const double xe = lx[0][wr + 1], xv = lx[0][wr], xn = lx[0][nn], xs = lx[0][sn];
+            cr.x = cr.x + omega * cr.over_ac(cr.res(xe, xv, xn, xs));
+            lx[1][tid] = cr.x;
+            if (cr.out) {
+                const double rv = cr.res(xe, xv, xn, xs);
+                if (m < S2_K) acc[m] += rv * rv;
+            }
+        }
+        __syncthreads();
+    }
+    if (cb.out) dst[cb.cc] = cb.x;
+    if (cr.out) dst[cr.cc] = cr.x;
+    if (mrun < S2_K) return;
+    block_partials<S2_NT, S2_K>(acc, pout, &red[0][0]);
+}
+
+// a finished solve's x out of the buffer the last iteration left it in, and
+// its residual when the caller keeps one (repeating it changes nothing)
+template <class OP>
+__global__ __launch_bounds__(NT) void k_sor2d_out(Tiling tl, Geom g, OP a, double *x, const double *__restrict__ xw,
+                                                  const double *__restrict__ b, double *__restrict__ r,
+                                                  const DevState *st) {
+    if (!st->done) return;
+    const bool away = st->plast != 0;
+    for_each_cell(tl, [&](int i, int j, int k) {
+        const int cc = g.id(i, j, k);
+        const double *s = away ? xw : x;
+        if (r) {
+            double ac, aw, ae, as, an, ab, at;
+            a.get(cc, i, j, k, ac, aw, ae, as, an, ab, at);
+            // a ghost neighbour is the caller's
+            const auto at_ = [&](int ii, int jj, int c) {
+                return (ii < g.gc || ii >= g.nx - g.gc || jj < g.gc || jj >= g.ny - g.gc) ? x[c] : s[c];
+            };
+            r[cc] = b[cc] - (ac * s[cc] + ae * at_(i + 1, j, cc + 1) + aw * at_(i - 1, j, cc - 1) +
+                             an * at_(i, j + 1, cc + g.nx) + as * at_(i, j - 1, cc - g.nx) + at * x[cc + g.nxy] +
+                             ab * x[cc - g.nxy]);
+        }
+        if (away) x[cc] = xw[cc];
+    });
+}
+
 template <class TS, class TD>
 __global__ void k_convert(const TS *__restrict__ s, TD *__restrict__ d, size_t n) {
     for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
@@ -1537,6 +1784,7 @@ struct falm_solver {
     K7Tiling kt;   // k-marching column tiles of the interior (stencil kernels)
     K7Tiling ktp;  // the same for k_bicg_pcmv_km (its own chunk length)
     S3Tiling s3;   // tiles of the fused three-sweep SOR kernel
+    S2Tiling s2;   // tiles of the one-layer SOR solver
     DevState *st = nullptr;
     DevState *hst = nullptr;  // pinned mirror
     double *partials = nullptr;
@@ -1606,6 +1854,7 @@ static falm_status solver_alloc(falm_solver *S) {
     size_t nb = (size_t)(S->tl.tiles > 0 ? red_blocks(S->tl) : 1);
     if ((size_t)S->kt.blocks > nb) nb = (size_t)S->kt.blocks;
     if ((size_t)S->ktp.blocks > nb) nb = (size_t)S->ktp.blocks;
+    if ((size_t)S->s2.blocks * s2_k(S->s2) > 2 * nb) nb = (size_t)S->s2.blocks * s2_k(S->s2) / 2 + 1;  // k_sor2d's norms
     FALM_HIP(hipMalloc(&S->partials, 2 * nb * sizeof(double)));
     FALM_HIP(hipMalloc(&S->trash, (size_t)(S->ktp.blocks > 0 ? S->ktp.blocks : 1) * K7_NT * 2 * sizeof(double)));
     if (S->cfg.pc_type == FALM_LS_SOR && S->cfg.pc_maxit <= 1) {  // the fused path (deferred_pc)
@@ -2025,11 +2274,67 @@ static falm_status solve_bicgstab_mixed(falm_solver *S, const OP64 &a64, const O
     return FALM_OK;
 }
 
+// FalmEq::SOR on one interior layer (k_sor2d): launches of K iterations,
+// the host polling once a batch.  A solve of n iterations takes
+// ceil(n / K) + 1 launches; the first batch is the previous solve's number.
+template <class OP>
+static falm_status solve_sor2d(falm_solver *S, const OP &a, double *x, const double *b, double *r, hipStream_t s,
+                               falm_solve_info *info, int mode) {
+    const falm_solver_config &c = S->cfg;
+    int &L = S->cur_enqueued;
+    double *const rout = r == S->r64own ? nullptr : r;
+    const auto enqueue = [&](int n) -> falm_status {
+        for (int q = 0; q < n; q++, L++) {
+            const double *pin = (L & 1) ? S->partials : S->partials2;
+            double *pout = (L & 1) ? S->partials2 : S->partials;
+#define FALM_S2(C)                                                                                            \
+    hipLaunchKernelGGL((k_sor2d<OP, C>), dim3((unsigned)S->s2.blocks), dim3(C::NT), 0, s, S->s2, S->g, a, x,  \
+                       (double *)S->w, b, c.relax, S->st, pin, pout, L)
+            if (S->s2.cfg == 0) FALM_S2(S2A);
+            else if (S->s2.cfg == 1) FALM_S2(S2B);
+            else FALM_S2(S2C);
+#undef FALM_S2
+        }
+        hipLaunchKernelGGL((k_sor2d_out<OP>), FALM_GRID(S), s, S->tl, S->g, a, x, (const double *)S->w, b, rout,
+                           (const DevState *)S->st);
+        FALM_CHECK_LAUNCH("k_sor2d");
+        return FALM_OK;
+    };
+    const int K = s2_k(S->s2);
+    const int poll = (check_period(S) + K - 1) / K;
+    const int last = (c.maxit - 1) / K + 2;  // launches after which any solve is over
+    const auto batch = [&](int n) { return n < last - L ? n : last - L; };
+    if (mode != SOLVE_RESUME) {
+        hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(64), 0, s, S->st, interior_count(S), 0, c.tol, c.maxit,
+                           0.0, 0, 0);
+        FALM_CHECK_LAUNCH("k_state_reset");
+        L = 0;
+        const int want = S->last_it > 0 && c.check_every <= 0 ? (S->last_it - 1) / K + 2 : poll;
+        FALM_TRY(enqueue(batch(want < 1024 ? want : 1024)));
+        if (mode == SOLVE_BEGIN) return FALM_OK;
+    }
+    bool first_read = true;
+    while (true) {
+        FALM_TRY(read_state(S, s));
+        if (first_read) S->first_ok = S->hst->done;
+        first_read = false;
+        if (S->hst->done || L >= last) break;
+        FALM_TRY(enqueue(batch(poll)));
+    }
+    info->it = S->hst->it_pass;
+    info->err = S->hst->err;
+    info->outer_it = 1;
+    info->status = S->hst->err <= c.tol ? FALM_OK : FALM_ERR_NOT_CONVERGED;
+    S->last_it = info->it;
+    return FALM_OK;
+}
+
 // FalmEq::SOR (src/FalmEq.cpp:173-240) and FalmEq::Jacobi (:81-127)
 template <class OP>
 static falm_status solve_stationary(falm_solver *S, const OP &a, double *x, const double *b, double *r,
                                     hipStream_t s, falm_solve_info *info, int mode) {
     const falm_solver_config &c = S->cfg;
+    if (c.type == FALM_LS_SOR && S->s2.blocks > 0) return solve_sor2d(S, a, x, b, r, s, info, mode);
     const int period = check_period(S);
     const int *done = &S->st->done;
     const int nb = red_blocks(S->tl);
@@ -2307,6 +2612,7 @@ falm_status falm_solver_create(const falm_domain *dom, const falm_solver_config 
         if (!even || S->tl.tiles == 0) S->tp.tiles = 0;
     }
     S->s3 = make_s3_tiling(interior_box(S->g));
+    S->s2 = make_s2_tiling(interior_box(S->g));
     falm_status st = solver_alloc(S);
     if (st != FALM_OK) {
         falm_solver_destroy(S);

@@ -1,0 +1,80 @@
+"""The SOR solver on one interior layer (several iterations a launch, stopped
+in the middle of a launch, at its end and by maxit) against the oracle's
+sweeps: the same iterations, the same x and residual.  Both apply the same
+expression cell by cell; only fused multiply-adds differ, 1e-12 after tens of
+contracting sweeps."""
+import numpy as np
+import pytest
+
+from falm_amd import _abi as abi
+from oracle import pyoracle as O
+from tests.helpers import domain, from_dev, interior_mask, rel_err, to_dev, uniform_metrics
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(n, gc, offset, seed):
+    dom = domain(n, gc=gc, offset=offset, gshape=tuple(v + 2 * gc + o for v, o in zip(n, offset)))
+    d0 = domain(n, gc=gc)
+    _, (_, _, g, ja) = uniform_metrics(d0, stretch=0.01)
+    a, _ = O.poisson_matrix(d0, abi.POISSON_OUTLET_XPLUS, g, ja)
+    rng = np.random.default_rng(seed)
+    # couplings to the ghost layers above and below, and ghost values, which stay as they are
+    m = interior_mask(dom)
+    nc = dom.ncell
+    for c in (5, 6):
+        a[c * nc:(c + 1) * nc] = np.where(m, 0.01 * rng.standard_normal(nc), 0.0)
+    return dom, a, rng.standard_normal(nc), rng.standard_normal(nc) * m, m
+
+
+# one cell; a 12 x 12 tile (7 iterations a launch) less, exactly and more than
+# full; several tiles and more guide cells; the colour shifted by an offset;
+# beyond 128 such tiles (16 x 16, 6 a launch), beyond 128 of those (32 x 16, 4)
+# and beyond 256 of those (separate sweeps)
+@pytest.mark.parametrize("n,gc,offset", [((1, 1, 1), 2, (0, 0, 0)), ((11, 11, 1), 2, (0, 0, 0)),
+                                         ((12, 12, 1), 2, (0, 0, 0)), ((13, 25, 1), 2, (0, 0, 0)),
+                                         ((100, 50, 1), 3, (0, 0, 0)), ((66, 35, 1), 2, (1, 0, 0)),
+                                         ((133, 145, 1), 2, (0, 0, 0)), ((300, 130, 1), 2, (0, 1, 0)),
+                                         ((520, 257, 1), 2, (0, 0, 0))])
+@pytest.mark.parametrize("declared", [False, True])
+def test_sor_one_layer(gpu, n, gc, offset, declared):
+    dom, a, x0, b, m = _system(n, gc, offset, 3)
+    da, db = to_dev(a), to_dev(b)
+    # (one cell's residual reaches rounding, where the stop is arbitrary, by 45)
+    for maxit in (1, 3, 4, 5, 6, 7, 8, 14) + ((45,) if m.sum() > 1 else ()):
+        cfg = abi.solver_config(type=abi.LS_SOR, maxit=maxit, tol=1e-30, relax=1.3, pc_type=abi.LS_EMPTY)
+        x_ref, r_ref = x0.copy(), np.zeros(dom.ncell)
+        i_ref = O.Solver(dom, cfg).solve(a, x_ref, b, r_ref)
+        S = gpu.Solver(dom, cfg)
+        if declared:
+            S.set_matrix(da)
+        dx, dr = to_dev(x0), to_dev(np.zeros(dom.ncell))
+        info = S.solve(da, dx, db, dr)
+        assert info.it == i_ref.it == maxit and info.status == i_ref.status, maxit
+        got = from_dev(dx)
+        assert rel_err(got, x_ref) < 1e-12, maxit
+        assert np.array_equal(got[~m], x0[~m])  # ghosts untouched
+        # the residual's rounding is that of x and b, not of itself
+        assert np.max(np.abs(from_dev(dr) - r_ref)[m]) < 1e-12 * np.max(np.abs(b)), maxit
+        assert abs(info.err - i_ref.err) <= 1e-9 * i_ref.err, maxit
+
+
+def test_sor_one_layer_stops_and_goes_on(gpu):
+    """The stop test's iteration, solve after solve on one handle (the first
+    batch is the previous solve's length), and without a residual."""
+    dom, a, x0, b, m = _system((100, 50, 1), 2, (0, 0, 0), 5)
+    da, db = to_dev(a), to_dev(b)
+    S = None
+    for tol, with_r in ((1e-3, True), (4e-4, False), (2e-3, True), (1e-3, True), (7e-4, False)):
+        cfg = abi.solver_config(type=abi.LS_SOR, maxit=2000, tol=tol, relax=1.5, pc_type=abi.LS_EMPTY)
+        x_ref, r_ref = x0.copy(), np.zeros(dom.ncell)
+        i_ref = O.Solver(dom, cfg).solve(a, x_ref, b, r_ref)
+        if S is None:
+            S = gpu.Solver(dom, cfg)
+        one = S if tol == 1e-3 else gpu.Solver(dom, cfg)
+        for _ in range(2):
+            dx = to_dev(x0)
+            dr = to_dev(np.zeros(dom.ncell)) if with_r else None
+            info = one.solve(da, dx, db, dr)
+            assert info.it == i_ref.it and info.status == i_ref.status == abi.FALM_OK, tol
+            assert rel_err(from_dev(dx), x_ref) < 1e-10
