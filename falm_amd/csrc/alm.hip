@@ -8,8 +8,8 @@
 //   is separable on the tensor-product grid, exp(-r^2/eps^2) =
 //   ex(x_i) ey(y_j) ez(z_k), so each point's three 1-D factor rows are
 //   evaluated once per step and a cell-point pair costs two products
-//   instead of an exp.  A fixed grid walks 32x8-cell tiles of the force box
-//   (of the whole interior on a full write); each tile first culls, in LDS,
+//   instead of an exp.  A fixed grid walks 32x2-cell tiles of the force box
+//   (on a full write k_alm_zero clears the rest); each tile first culls, in LDS,
 //   the points whose kernel value is exactly zero in double precision over
 //   the whole tile (r^2/eps^2 > 746), keeping the survivors in ascending id
 //   order; a finite cutoff (radius in units of eps) culls harder.
@@ -331,16 +331,20 @@ __global__ __launch_bounds__(256) void k_alm_points(AlmDev A, const T *u0, const
     if (!fused) return;
     __syncthreads();
     alm_box_wg(A, sxyz, X, Y, Z);
-    // k_alm_totals: per-turbine sums in ascending point order
-    if ((int)threadIdx.x < A.nt) {
-        const int napt = A.napb * A.nb, tid = threadIdx.x;
+    // k_alm_totals: per-turbine sums, one turbine to a wave at a time
+    const int napt2 = A.napb * A.nb;
+    for (int tb = threadIdx.x >> 6; tb < A.nt; tb += 4) {
         double tq = 0.0, th = 0.0;
-        for (int a = 0; a < napt; a++) {
-            tq += stq[tid * napt + a];
-            th += sth[tid * napt + a];
+        for (int a = threadIdx.x & 63; a < napt2; a += 64) {
+            tq += stq[tb * napt2 + a];
+            th += sth[tb * napt2 + a];
         }
-        A.torque[tid] = tq;
-        A.thrust[tid] = th;
+        tq = wave_sum(tq);
+        th = wave_sum(th);
+        if ((threadIdx.x & 63) == 0) {
+            A.torque[tb] = tq;
+            A.thrust[tb] = th;
+        }
     }
 }
 
@@ -358,10 +362,8 @@ __device__ void alm_box_wg(const AlmDev &A, const double *pxyz, const double *X,
             mx[m] = fmax(mx[m], pxyz[3 * ap + m]);
         }
     for (int m = 0; m < 3; m++) {
-        for (int off = 32; off > 0; off >>= 1) {
-            mn[m] = fmin(mn[m], __shfl_down(mn[m], off, 64));
-            mx[m] = fmax(mx[m], __shfl_down(mx[m], off, 64));
-        }
+        mn[m] = wave_reduce(mn[m], [](double p, double q) { return fmin(p, q); });
+        mx[m] = wave_reduce(mx[m], [](double p, double q) { return fmax(p, q); });
         if (lane == 0) {
             smn[m][wid] = mn[m];
             smx[m][wid] = mx[m];
@@ -392,10 +394,8 @@ __device__ void alm_box_wg(const AlmDev &A, const double *pxyz, const double *X,
                 hi[m] = max(hi[m], i);
             }
         }
-        for (int off = 32; off > 0; off >>= 1) {
-            lo[m] = min(lo[m], __shfl_down(lo[m], off, 64));
-            hi[m] = max(hi[m], __shfl_down(hi[m], off, 64));
-        }
+        lo[m] = wave_reduce(lo[m], [](int p, int q) { return min(p, q); });
+        hi[m] = wave_reduce(hi[m], [](int p, int q) { return max(p, q); });
         if (lane == 0) {
             slo[m][wid] = lo[m];
             shi[m][wid] = hi[m];
@@ -451,15 +451,16 @@ constexpr int PJ_W = 4;             // waves per workgroup, each summing a share
 
 // The Gaussian projection, walking the tiles of the cells it writes with a
 // fixed grid: the union of this and the previous step's force box
-// (union_only; ff is zero elsewhere and stays untouched), or every interior
-// cell.  Cells outside this step's box get zero.  Per tile, the points whose
+// (union_only; ff is zero elsewhere and stays untouched), or this step's box
+// (k_alm_zero writes the other interior cells).  Cells outside this step's box
+// get zero.  Per tile, the points whose
 // Gaussian reaches the tile within the culling radius are compacted into
 // LDS with their per-axis factors; each of the four waves sums a contiguous
 // quarter of them for the tile's 64 cells, and the quarters are added in
 // wave order.  A box of a few tens of thousands of cells then keeps four
 // waves busy per tile instead of one.
 template <class T>
-__global__ __launch_bounds__(256) void k_alm_project(Box interior, AlmDev A, T *ff0, T *ff1, T *ff2, double cut2,
+__global__ __launch_bounds__(256) void k_alm_project(AlmDev A, T *ff0, T *ff1, T *ff2, double cut2,
                                                      int union_only) {
     static_assert(PJ_X * PJ_Y == 64 && PJ_W * 64 == 256, "one tile cell per lane, four waves");
     __shared__ double sf0[kCullChunk], sf1[kCullChunk], sf2[kCullChunk], sez[kCullChunk];
@@ -468,18 +469,11 @@ __global__ __launch_bounds__(256) void k_alm_project(Box interior, AlmDev A, T *
     __shared__ double part[PJ_W - 1][3][64];
     __shared__ int wcount[PJ_W];
     int wlo[3], wn[3];
-    if (union_only) {
-        const int *U = A.box + 6;
-        if (U[0] > U[1]) return;
-        for (int m = 0; m < 3; m++) {
-            wlo[m] = U[2 * m];
-            wn[m] = U[2 * m + 1] - U[2 * m] + 1;
-        }
-    } else {
-        for (int m = 0; m < 3; m++) {
-            wlo[m] = interior.lo[m];
-            wn[m] = interior.n[m];
-        }
+    const int *U = union_only ? A.box + 6 : A.box;
+    if (U[0] > U[1]) return;
+    for (int m = 0; m < 3; m++) {
+        wlo[m] = U[2 * m];
+        wn[m] = U[2 * m + 1] - U[2 * m] + 1;
     }
     const int tx = (wn[0] + PJ_X - 1) / PJ_X, ty = (wn[1] + PJ_Y - 1) / PJ_Y;
     const long long ntiles = (long long)tx * ty * wn[2];
@@ -580,6 +574,23 @@ __global__ __launch_bounds__(256) void k_alm_project(Box interior, AlmDev A, T *
         }
         __syncthreads();
     }
+}
+
+// The interior cells outside this step's force box, on a full write: zero.
+// A stream of stores, one tile a workgroup: the projection's own walk over all
+// tiles of the interior, where one wave in four writes such a tile, took 101
+// us for 384 x 128 x 128 cells in double (151 MB); box and stream take 25 + 22 us.
+template <class T>
+__global__ __launch_bounds__(256) void k_alm_zero(Tiling tl, Geom g, AlmDev A, T *ff0, T *ff1, T *ff2) {
+    const int *B = A.box;
+    const int b0 = B[0], b1 = B[1], b2 = B[2], b3 = B[3], b4 = B[4], b5 = B[5];
+    for_each_cell(tl, [&](int i, int j, int k) {
+        if (i >= b0 && i <= b1 && j >= b2 && j <= b3 && k >= b4 && k <= b5) return;
+        const int c = g.id(i, j, k);
+        ff0[c] = T(0);
+        ff1[c] = T(0);
+        ff2[c] = T(0);
+    });
 }
 
 // per-turbine sums in ascending point order; the point values are first
@@ -1091,16 +1102,21 @@ falm_status alm_step(falm_alm *A, int prec, const void *u, void *ff, double t, h
     hipLaunchKernelGGL(k_alm_factors, dim3((nfac + 255) / 256), dim3(256), 0, s, A->d);
     FALM_CHECK_LAUNCH("k_alm_factors");
     if (tl.tiles > 0) {
-        // enough workgroups for a force box; a full write walks its tiles
+        // enough workgroups for a force box
         const Box ib = interior_box(g);
         const long long full = (long long)((ib.n[0] + PJ_X - 1) / PJ_X) * ((ib.n[1] + PJ_Y - 1) / PJ_Y) * ib.n[2];
         const dim3 grid((unsigned)(full < 2048 ? full : 2048));
-        if (prec == FALM_F32)
-            hipLaunchKernelGGL((k_alm_project<float>), grid, dim3(256), 0, s, ib, A->d, col<float>(ff, n, 0),
-                               col<float>(ff, n, 1), col<float>(ff, n, 2), A->cut2, union_only);
-        else
-            hipLaunchKernelGGL((k_alm_project<double>), grid, dim3(256), 0, s, ib, A->d, col<double>(ff, n, 0),
-                               col<double>(ff, n, 1), col<double>(ff, n, 2), A->cut2, union_only);
+#define FALM_PROJECT(T)                                                                                          \
+    do {                                                                                                         \
+        if (!union_only)                                                                                         \
+            hipLaunchKernelGGL((k_alm_zero<T>), tiling_grid(tl), tiling_block(), 0, s, tl, g, A->d,              \
+                               col<T>(ff, n, 0), col<T>(ff, n, 1), col<T>(ff, n, 2));                            \
+        hipLaunchKernelGGL((k_alm_project<T>), grid, dim3(256), 0, s, A->d, col<T>(ff, n, 0), col<T>(ff, n, 1),  \
+                           col<T>(ff, n, 2), A->cut2, union_only);                                               \
+    } while (0)
+        if (prec == FALM_F32) FALM_PROJECT(float);
+        else FALM_PROJECT(double);
+#undef FALM_PROJECT
         FALM_CHECK_LAUNCH("k_alm_project");
     }
     if (!fused) hipLaunchKernelGGL(k_alm_totals, dim3(A->nt), dim3(256), 0, s, A->d);

@@ -254,6 +254,31 @@ __device__ inline double wave_sum(double v) {
     return __hiloint2double(hi, lo);
 }
 
+// Wavefront minimum / maximum through the same moves (a lane that receives
+// nothing keeps its own value); every lane gets it.
+template <int CTRL, int ROWS>
+__device__ inline int dpp_or_own(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ inline double dpp_or_own(double v) {
+    return __hiloint2double(dpp_or_own<CTRL, ROWS>(__double2hiint(v)), dpp_or_own<CTRL, ROWS>(__double2loint(v)));
+}
+__device__ inline int lane63(int v) { return __builtin_amdgcn_readlane(v, 63); }
+__device__ inline double lane63(double v) {
+    return __hiloint2double(lane63(__double2hiint(v)), lane63(__double2loint(v)));
+}
+template <class V, class F>
+__device__ inline V wave_reduce(V v, F f) {
+    v = f(v, dpp_or_own<0x111, 0xf>(v));
+    v = f(v, dpp_or_own<0x112, 0xf>(v));
+    v = f(v, dpp_or_own<0x114, 0xf>(v));
+    v = f(v, dpp_or_own<0x118, 0xf>(v));
+    v = f(v, dpp_or_own<0x142, 0xa>(v));
+    v = f(v, dpp_or_own<0x143, 0xc>(v));
+    return lane63(v);
+}
+
 // Multi-value block sum (NV values per thread): every wave's sums go to LDS
 // (lds holds NV * NT/64), and wave q sums value q's NT/64 of them, so that the
 // values are summed side by side and not one after the other in one thread.
