@@ -424,6 +424,164 @@ __global__ __launch_bounds__(KM_NT) void k_pseudo_u_km(KmTiling kt, Geom g, T Re
     }
 }
 
+// The C-ABI pseudo-velocity (per-cell metric fields) in k-marching form.  A
+// cell costs 31 vector loads instead of the 71 of k_pseudo_u: u (two-cell halo)
+// and nut (one-cell halo) come from LDS planes and register queues, the face
+// flux and g along z from the previous plane's registers, g's x and y
+// neighbours and the other fluxes from cache lines of the row.  The arithmetic
+// is k_pseudo_u's, expression by expression.  512 x 128 x 128 in double: 461 ->
+// 340 us (1.54 GB of operands, 4.5 TB/s).
+template <int SCHEME, class T>
+__global__ __launch_bounds__(KM_NT) void k_pseudo_u_fm(KmTiling kt, Geom g, T ReI, T dt, Vec3<T> un, Vec3<T> u,
+                                                       Vec3<T> uu, Vec3W<T> ua, const T *__restrict__ nut,
+                                                       MetField<T> met, Vec3<T> ff) {
+    constexpr unsigned TS = sizeof(T);
+    __shared__ T su[2][3][KM_BY + 4][KM_BX + 4];
+    __shared__ T sn[2][KM_BY + 2][KM_BX + 2];
+    const int lane = threadIdx.x & (KM_BX - 1);
+    const int wy = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / KM_BX));
+    const int L = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x));
+    const int bx = L % kt.tx, by = (L / kt.tx) % kt.ty, kc = L / (kt.tx * kt.ty);
+    const int i0 = kt.box.lo[0] + bx * KM_BX, j0 = kt.box.lo[1] + by * KM_BY;
+    const int i = i0 + lane, j = j0 + wy;
+    const bool act = i < kt.box.lo[0] + kt.box.n[0] && j < kt.box.lo[1] + kt.box.n[1];
+    const int k0 = kt.box.lo[2] + kc * kt.kc;
+    const int k1 = min(k0 + kt.kc, kt.box.lo[2] + kt.box.n[2]);
+    const int sy = g.nx;
+    const unsigned syb = (unsigned)sy * TS, szb = (unsigned)g.nxy * TS;
+    // as in k_pseudo_u_km: threads past the box load their own cell into the
+    // planes when it lies in the array, and compute (without storing) on the
+    // box's first column
+    const bool ld = i < g.nx && j < g.ny;
+    const unsigned col = (unsigned)((ld ? i : kt.box.lo[0]) + sy * (ld ? j : kt.box.lo[1])) * TS;
+    const unsigned own = (unsigned)((act ? i : kt.box.lo[0]) + sy * (act ? j : kt.box.lo[1])) * TS;
+    const T *hp[KM_HPT];
+    int hl[KM_HPT];
+    bool hok[KM_HPT], hu[KM_HPT];
+#pragma unroll
+    for (int q = 0; q < KM_HPT; q++) {
+        const int s = threadIdx.x + q * KM_NT;
+        int arr = 3, row = 0, c = 0;
+        if (s < KM_HALO) km_halo_slot(s, arr, row, c);
+        const int gi = i0 - (arr < 3 ? 2 : 1) + c, gj = j0 - (arr < 3 ? 2 : 1) + row;
+        hu[q] = s < KM_HALO;
+        hok[q] = hu[q] && gi >= 0 && gi < g.nx && gj >= 0 && gj < g.ny;
+        const T *src = arr == 0 ? u.c[0] : arr == 1 ? u.c[1] : arr == 2 ? u.c[2] : nut;
+        hp[q] = hok[q] ? src + gi + sy * gj : reinterpret_cast<const T *>(reinterpret_cast<const char *>(src) + col);
+        hl[q] = arr < 3 ? (int)(&su[0][arr][row][c] - &su[0][0][0][0]) : -1 - (int)(&sn[0][row][c] - &sn[0][0][0]);
+    }
+    auto halo_load = [&](int k, T (&hv)[KM_HPT]) {
+#pragma unroll
+        for (int q = 0; q < KM_HPT; q++) {
+            const T v = hp[q][(size_t)g.nxy * k];
+            hv[q] = hok[q] ? v : T(0);
+        }
+    };
+    auto lds_fill = [&](int b, const T (&hv)[KM_HPT], T u0, T u1, T u2, T nv) {
+        su[b][0][wy + 2][lane + 2] = u0;
+        su[b][1][wy + 2][lane + 2] = u1;
+        su[b][2][wy + 2][lane + 2] = u2;
+        sn[b][wy + 1][lane + 1] = nv;
+#pragma unroll
+        for (int q = 0; q < KM_HPT; q++) {
+            if (!hu[q]) continue;
+            if (hl[q] >= 0) (&su[b][0][0][0])[hl[q]] = hv[q];
+            else (&sn[b][0][0])[-1 - hl[q]] = hv[q];
+        }
+    };
+    // a plane's own operands, loaded a plane ahead
+    struct Op {
+        T uu[5], gx[3], gy[3], gzt, kx[3], ja, un[3], ff[3];
+    };
+    const auto load = [&](int k) {
+        const unsigned c = own + (unsigned)k * szb;
+        Op o;
+        o.uu[0] = ld_at(uu.c[0], c);
+        o.uu[1] = ld_at(uu.c[0], c - TS);
+        o.uu[2] = ld_at(uu.c[1], c);
+        o.uu[3] = ld_at(uu.c[1], c - syb);
+        o.uu[4] = ld_at(uu.c[2], c);
+        o.gx[0] = ld_at(met.g[0], c - TS);
+        o.gx[1] = ld_at(met.g[0], c);
+        o.gx[2] = ld_at(met.g[0], c + TS);
+        o.gy[0] = ld_at(met.g[1], c - syb);
+        o.gy[1] = ld_at(met.g[1], c);
+        o.gy[2] = ld_at(met.g[1], c + syb);
+        o.gzt = ld_at(met.g[2], c + szb);
+        o.ja = ld_at(met.ja, c);
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            o.kx[d] = ld_at(met.kx[d], c);
+            o.un[d] = ld_at(un.c[d], c);
+            o.ff[d] = ld_at(ff.c[d], c);
+        }
+        return o;
+    };
+    T qu[3][5], qn[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int d = 0; d < 5; d++) qu[c][d] = ld_at(u.c[c], col + (unsigned)(k0 - 2 + d) * szb);
+#pragma unroll
+    for (int d = 0; d < 3; d++) qn[d] = ld_at(nut, col + (unsigned)(k0 - 1 + d) * szb);
+    T wb = ld_at(uu.c[2], own + (unsigned)(k0 - 1) * szb);
+    T gzb = ld_at(met.g[2], own + (unsigned)(k0 - 1) * szb), gzc = ld_at(met.g[2], own + (unsigned)k0 * szb);
+    Op nx = load(k0);
+    T hv[KM_HPT];
+    halo_load(k0, hv);
+    lds_fill(0, hv, qu[0][2], qu[1][2], qu[2][2], qn[1]);
+    __syncthreads();
+    int b = 0;
+    for (int k = k0; k < k1; k++) {
+        const bool more = k + 1 < k1;
+        const Op o = nx;
+        T nu[3] = {T(0), T(0), T(0)}, nn = T(0);
+        if (more) {  // loads for plane k+1
+            halo_load(k + 1, hv);
+#pragma unroll
+            for (int c = 0; c < 3; c++) nu[c] = ld_at(u.c[c], col + (unsigned)(k + 3) * szb);
+            nn = ld_at(nut, col + (unsigned)(k + 2) * szb);
+            nx = load(k + 1);
+        }
+        const T rjac = T(1) / o.ja;
+        const T Uabs = fabs(qu[0][2] * o.kx[0]), Vabs = fabs(qu[1][2] * o.kx[1]), Wabs = fabs(qu[2][2] * o.kx[2]);
+        const T UE = o.uu[0], UW = o.uu[1], VN = o.uu[2], VS = o.uu[3], WT = o.uu[4], WB = wb;
+        const T nc = qn[1], ne = sn[b][wy + 1][lane + 2], nw = sn[b][wy + 1][lane], nn1 = sn[b][wy + 2][lane + 1],
+                ns = sn[b][wy][lane + 1], nt = qn[2], nb = qn[0];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const T ucc = qu[d][2];
+            const T ue1 = su[b][d][wy + 2][lane + 3], ue2 = su[b][d][wy + 2][lane + 4];
+            const T uw1 = su[b][d][wy + 2][lane + 1], uw2 = su[b][d][wy + 2][lane];
+            const T un1 = su[b][d][wy + 3][lane + 2], un2 = su[b][d][wy + 4][lane + 2];
+            const T us1 = su[b][d][wy + 1][lane + 2], us2 = su[b][d][wy][lane + 2];
+            const T ut1 = qu[d][3], ut2 = qu[d][4], ub1 = qu[d][1], ub2 = qu[d][0];
+            const T adv = advection<SCHEME, T>(ucc, ue1, ue2, uw1, uw2, un1, un2, us1, us2, ut1, ut2, ub1, ub2, Uabs,
+                                               Vabs, Wabs, UE, UW, VN, VS, WT, WB, rjac);
+            const T vis = diffusion<T>(ReI, ucc, ue1, uw1, un1, us1, ut1, ub1, nc, ne, nw, nn1, ns, nt, nb, o.gx[1],
+                                       o.gx[2], o.gx[0], o.gy[1], o.gy[2], o.gy[0], gzc, o.gzt, gzb, rjac);
+            if (act) st_at(ua.c[d], own + (unsigned)k * szb, o.un[d] + dt * (-adv + vis + o.ff[d]));
+        }
+        if (more) lds_fill(b ^ 1, hv, qu[0][3], qu[1][3], qu[2][3], qn[2]);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            qu[c][0] = qu[c][1];
+            qu[c][1] = qu[c][2];
+            qu[c][2] = qu[c][3];
+            qu[c][3] = qu[c][4];
+            qu[c][4] = nu[c];
+        }
+        qn[0] = qn[1];
+        qn[1] = qn[2];
+        qn[2] = nn;
+        wb = WT;
+        gzb = gzc;
+        gzc = o.gzt;
+        b ^= 1;
+        __syncthreads();
+    }
+}
+
 // Device view of the coefficient tables in one precision.
 template <class T>
 struct SepTab {
@@ -1191,6 +1349,66 @@ __global__ __launch_bounds__(K7_NT) void k_sgs_div_km(K7Tiling kt, Geom g, T Cs,
     block_partials<K7_NT, 1>(v, partials, lds);
 }
 
+// k_smagorinsky as the step driver's kernel walks it, with the metric fields
+// read instead of the tables (the C-ABI operation on large domains); the
+// expressions are k_smagorinsky's.  512 x 128 x 128 in double: 154 -> 131 us (537 MB, 4.1 TB/s;
+// the square and cube roots take about 30 us of it).  The projection walked
+// the same way measured 309 us against k_project's 291, so it stays a thread
+// per cell.
+template <class T>
+__global__ __launch_bounds__(K7_NT) void k_smagorinsky_fm(K7Tiling kt, Geom g, T Cs, Vec3<T> u, T *__restrict__ nut,
+                                                          MetField<T> met) {
+    __shared__ K7Lds<T> l0, l1, l2;
+    const K7Pos Q = k7_pos(kt, g);
+    const int sz = g.nxy;
+    const unsigned szb = (unsigned)sz * sizeof(T);
+    Plane7<T> pu[3];
+    pu[0].setup(u.c[0], &l0, Q, g);
+    pu[1].setup(u.c[1], &l1, Q, g);
+    pu[2].setup(u.c[2], &l2, Q, g);
+#pragma unroll
+    for (int d = 0; d < 3; d++) pu[d].prologue(Q, sz);
+    unsigned cb = (unsigned)Q.col0 * sizeof(T) + (unsigned)Q.k0 * szb;
+    T kn[3], jn = ld_at(met.ja, cb);
+#pragma unroll
+    for (int d = 0; d < 3; d++) kn[d] = ld_at(met.kx[d], cb);
+    __syncthreads();
+    int b = 0;
+    for (int k = Q.k0; k < Q.k1; k++, cb += szb) {
+        const bool more = k + 1 < Q.k1;
+        const T kxx = kn[0], kxy = kn[1], kxz = kn[2], J = jn;
+        if (more) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                pu[d].prefetch(Q, k, sz);
+                kn[d] = ld_at(met.kx[d], cb + szb);
+            }
+            jn = ld_at(met.ja, cb + szb);
+        }
+        if (Q.act) {
+            T gr[3][3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                gr[d][0] = T(0.5) * kxx * (pu[d].xp(b) - pu[d].xm(b));
+                gr[d][1] = T(0.5) * kxy * (pu[d].yp(b) - pu[d].ym(b));
+                gr[d][2] = T(0.5) * kxz * (pu[d].zp() - pu[d].zm());
+            }
+            const T dux = gr[0][0], duy = gr[0][1], duz = gr[0][2];
+            const T dvx = gr[1][0], dvy = gr[1][1], dvz = gr[1][2];
+            const T dwx = gr[2][0], dwy = gr[2][1], dwz = gr[2][2];
+            T d1 = T(2) * dux * dux, d2 = T(2) * dvy * dvy, d3 = T(2) * dwz * dwz;
+            T d4 = (duy + dvx) * (duy + dvx), d5 = (dvz + dwy) * (dvz + dwy), d6 = (duz + dwx) * (duz + dwx);
+            const T Du = sqrt(d1 + d2 + d3 + d4 + d5 + d6);
+            const T lc = Cs * cbrt(J);
+            st_at(nut, cb, lc * lc * Du);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++) pu[d].advance(b, more);
+        b ^= 1;
+        __syncthreads();
+    }
+}
+
 // hout (may be null): a pinned host copy of the result
 __global__ __launch_bounds__(FIN_NT) void k_fin_norm(const double *partials, int nb, double *out, const int *gate,
                                                      double *hout) {
@@ -1305,6 +1523,53 @@ static falm_status pseudo_u_t(const falm_domain *dom, int scheme, double ReI, do
     return FALM_OK;
 }
 
+// Whether a C-ABI operation with per-cell metric fields takes its k-marching
+// form: where a column stays below 4 GiB (32-bit byte offsets) and from 2 M
+// interior cells on.  Below, a thread per cell is as fast or faster (its loads
+// hit the caches, and its grid fills the chip): predictor of 133 x 67 x 45
+// cells in float 23 us against 26, 200 x 100 x 90 in float 59 us both, 256 x 96
+// x 96 in double 180 us against 164, 512 x 128 x 128 652 us against 548.
+constexpr long long FM_CELLS = 2000000;
+static bool marches(const Geom &g, size_t ncell, size_t elem) {
+    return interior_box(g).size() >= FM_CELLS && ncell * elem < (size_t(1) << 32);
+}
+
+// The C-ABI pseudo-velocity.
+template <class T>
+static falm_status pseudo_u_field_t(const falm_domain *dom, int scheme, double ReI, double dt, const void *un,
+                                    const void *u, const void *uu, void *ua, const void *nut, const MetField<T> &met,
+                                    const void *ff, hipStream_t s) {
+    const Geom g = make_geom(dom);
+    const size_t n = ncell_of(dom);
+    KmTiling kt = make_km_tiling(interior_box(g));
+    if (kt.blocks == 0) return FALM_OK;
+    // one round: two workgroups a CU in float, one in double (180 VGPRs); 512
+    // x 128 x 128 in double 548 us a predictor with two chunks of 64 planes,
+    // 574 with eight of 16
+    int tk = (sizeof(T) == 4 ? 2 : 1) * 256 / (kt.tx * kt.ty);
+    if (tk < 1) tk = 1;
+    kt.kc = (kt.box.n[2] + tk - 1) / tk;
+    kt.tk = (kt.box.n[2] + kt.kc - 1) / kt.kc;
+    kt.blocks = kt.tx * kt.ty * kt.tk;
+    if (!marches(g, n, sizeof(T)))
+        return pseudo_u_t<T>(dom, scheme, ReI, dt, un, u, uu, ua, nut, met, ff, nullptr, 23.0, s);
+    TimedLaunch tm(FALM_TIME_PSEUDO_U, s);
+#define FALM_PUF(S)                                                                                              \
+    hipLaunchKernelGGL((k_pseudo_u_fm<S, T>), dim3(kt.blocks), dim3(KM_NT), 0, s, kt, g, (T)ReI, (T)dt,          \
+                       v3<T>(un, n), v3<T>(u, n), v3<T>(uu, n), v3w<T>(ua, n), (const T *)nut, met, v3<T>(ff, n))
+    switch (scheme) {
+    case FALM_ADV_UPWIND3: FALM_PUF(FALM_ADV_UPWIND3); break;
+    case FALM_ADV_QUICK: FALM_PUF(FALM_ADV_QUICK); break;
+    case FALM_ADV_UTOPIA: FALM_PUF(FALM_ADV_UTOPIA); break;
+    case FALM_ADV_KK: FALM_PUF(FALM_ADV_KK); break;
+    default: FALM_PUF(FALM_ADV_UPWIND1); break;  // str2advscheme's fallback (src/FalmCFD.h:111-125)
+    }
+#undef FALM_PUF
+    FALM_CHECK_LAUNCH("k_pseudo_u_fm");
+    tm.done((double)interior_box(g).size() * 23.0 * sizeof(T));
+    return FALM_OK;
+}
+
 template <class T, class M>
 static falm_status u_to_uu_t(const falm_domain *dom, const void *u, void *uu, const M &met, hipStream_t s) {
     Geom g = make_geom(dom);
@@ -1370,6 +1635,22 @@ static falm_status smag_t(const falm_domain *dom, double Cs, const void *u, void
     FALM_CHECK_LAUNCH("k_smagorinsky");
     // u read, nut written (+ kx, ja)
     tm.done((double)tl.box.size() * (4.0 + (M::per_cell ? 4.0 : 0.0)) * sizeof(T));
+    return FALM_OK;
+}
+
+// the C-ABI Smagorinsky model (marches above)
+template <class T>
+static falm_status smag_field_t(const falm_domain *dom, double Cs, const void *u, void *nut, const MetField<T> &met,
+                                hipStream_t s) {
+    const Geom g = make_geom(dom);
+    const size_t n = ncell_of(dom);
+    if (!marches(g, n, sizeof(T))) return smag_t<T>(dom, Cs, u, nut, met, s);
+    const K7Tiling kt = make_k7_tiling_fit(interior_box(g), 512);  // one round, two a CU (88 VGPRs in double)
+    TimedLaunch tm(FALM_TIME_SGS, s);
+    hipLaunchKernelGGL((k_smagorinsky_fm<T>), dim3(kt.blocks), dim3(K7_NT), 0, s, kt, g, (T)Cs, v3<T>(u, n),
+                       (T *)nut, met);
+    FALM_CHECK_LAUNCH("k_smagorinsky_fm");
+    tm.done((double)interior_box(g).size() * 8.0 * sizeof(T));
     return FALM_OK;
 }
 
@@ -1595,10 +1876,10 @@ falm_status falm_pseudo_u(const falm_domain *dom, int prec, int adv_scheme, doub
     hipStream_t s = (hipStream_t)stream;
     const size_t n = ncell_of(dom);
     if (prec == FALM_F32)
-        return pseudo_u_t<float>(dom, adv_scheme, ReI, dt, un, u, uu, ua, nut, met_field<float>(kx, g, ja, n), ff,
-                                 nullptr, 23.0, s);
-    return pseudo_u_t<double>(dom, adv_scheme, ReI, dt, un, u, uu, ua, nut, met_field<double>(kx, g, ja, n), ff,
-                              nullptr, 23.0, s);
+        return pseudo_u_field_t<float>(dom, adv_scheme, ReI, dt, un, u, uu, ua, nut, met_field<float>(kx, g, ja, n),
+                                       ff, s);
+    return pseudo_u_field_t<double>(dom, adv_scheme, ReI, dt, un, u, uu, ua, nut, met_field<double>(kx, g, ja, n), ff,
+                                    s);
 }
 
 falm_status falm_u_to_uu(const falm_domain *dom, int prec, const void *u, void *uu, const void *kx,
@@ -1657,8 +1938,8 @@ falm_status falm_sgs(const falm_domain *dom, int prec, int model, double Cs, con
     }
     hipStream_t s = (hipStream_t)stream;
     const size_t n = ncell_of(dom);
-    if (prec == FALM_F32) return smag_t<float>(dom, Cs, u, nut, met_field<float>(kx, nullptr, ja, n), s);
-    return smag_t<double>(dom, Cs, u, nut, met_field<double>(kx, nullptr, ja, n), s);
+    if (prec == FALM_F32) return smag_field_t<float>(dom, Cs, u, nut, met_field<float>(kx, nullptr, ja, n), s);
+    return smag_field_t<double>(dom, Cs, u, nut, met_field<double>(kx, nullptr, ja, n), s);
 }
 
 falm_status falm_divergence(const falm_domain *dom, int prec, const void *uu, void *div, const void *ja,
