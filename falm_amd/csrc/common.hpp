@@ -364,8 +364,7 @@ template <class T> inline const T *col(const void *p, size_t ncell, int c) {
 // Library-owned device scratch for one-shot reductions (per device).
 struct ReduceScratch {
     double *partials = nullptr;  // 8 * max_blocks doubles
-    double *result = nullptr;    // 8 doubles
-    double *host = nullptr;      // pinned host mirror of result
+    double *host = nullptr;      // 8 doubles of pinned host memory, written by the finalize kernel
     size_t max_blocks = 0;
 };
 falm_status reduce_scratch(size_t nblocks, ReduceScratch **out);

@@ -34,24 +34,39 @@ template <class T, bool NORM>
 __global__ __launch_bounds__(256) void k_dot(Tiling tl, Geom g, const T *__restrict__ a, const T *__restrict__ b,
                                              int ncol, size_t ncell, double *partials) {
     __shared__ double lds[4];
-    int i, j, k, t0, t1;
+    int t0, t1;
     double v[1] = {0.0};
     tile_range(tl.tiles, t0, t1);
-    for (int tile = t0; tile < t1; tile++) {
-        if (!tile_cell_at(tl, tile, i, j, k)) continue;
-        const int cc = g.id(i, j, k);
-        if (NORM) {
-            for (int d = 0; d < ncol; d++) {
-                double x = (double)a[cc + d * ncell];
-                v[0] += x * x;
+    // four tiles at a time, every load issued before one is used (a cell past
+    // the box reads the box's first cell and adds nothing): a single tile's
+    // load leaves a wave waiting (squared norm in double at 512 x 128 x 128 21 ->
+    // 18 us, at 1024 x 256 x 256 133 -> 107 us)
+    const size_t c0 = (size_t)g.id(tl.box.lo[0], tl.box.lo[1], tl.box.lo[2]);
+    for (int tile = t0; tile < t1; tile += 4) {
+        size_t cc[4];
+        bool in[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            int i, j, k;
+            in[q] = tile + q < t1 && tile_cell_at(tl, tile + q, i, j, k);
+            cc[q] = in[q] ? (size_t)g.id(i, j, k) : c0;
+        }
+        for (int d = 0; d < (NORM ? ncol : 1); d++) {
+            double x[4], y[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                x[q] = (double)a[cc[q] + d * ncell];
+                y[q] = NORM ? x[q] : (double)b[cc[q]];
             }
-        } else {
-            v[0] += (double)a[cc] * (double)b[cc];
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[0] += in[q] ? x[q] * y[q] : 0.0;
         }
     }
     block_partials<256, 1>(v, partials, lds);
 }
 
+// out: device memory, or the pinned host memory that the caller reads after
+// its wait (no copy in between)
 __global__ __launch_bounds__(FIN_NT) void k_fin_sum(const double *partials, int nb, double *out) {
     double tot[1];
     sum_partials<1>(partials, nb, tot);
@@ -247,8 +262,7 @@ static falm_status host_scalar(const falm_domain *dom, int prec, const void *a, 
     Tiling tl = make_tiling(interior_box(g));
     ReduceScratch *rs;
     FALM_TRY(reduce_scratch((size_t)tl.tiles, &rs));
-    FALM_TRY(launch_dot(dom, prec, a, b, ncol, norm, rs->result, rs->partials, s));
-    FALM_HIP(hipMemcpyAsync(rs->host, rs->result, sizeof(double), hipMemcpyDeviceToHost, s));
+    FALM_TRY(launch_dot(dom, prec, a, b, ncol, norm, rs->host, rs->partials, s));
     FALM_HIP(hipStreamSynchronize(s));
     *out = rs->host[0];
     return FALM_OK;

@@ -65,10 +65,8 @@ falm_status reduce_scratch(size_t nblocks, ReduceScratch **out) {
         FALM_HIP(hipMalloc(&rs.partials, 8 * nb * sizeof(double)));
         rs.max_blocks = nb;
     }
-    if (!rs.result) {
-        FALM_HIP(hipMalloc(&rs.result, 8 * sizeof(double)));
-        FALM_HIP(hipHostMalloc(&rs.host, 8 * sizeof(double), hipHostMallocDefault));
-    }
+    // coherent: the finalize kernel writes it directly
+    if (!rs.host) FALM_HIP(hipHostMalloc(&rs.host, 8 * sizeof(double), hipHostMallocCoherent));
     *out = &rs;
     return FALM_OK;
 }
