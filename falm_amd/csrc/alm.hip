@@ -17,6 +17,8 @@
 //   uses thrust::reduce, src/alm/almDevCall.cu:362-370), kept on device.
 #include <cstddef>
 #include <cmath>
+#include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "alm.hpp"
@@ -1057,6 +1059,9 @@ struct falm_alm {
     double cut2;
     int nt, nap, napb;
     bool full_next = true;  // the next owned-ff step writes every cell
+    double *hout = nullptr;  // pinned copy of the block falm_alm_get returns, under mx
+    std::mutex mx;
+    size_t out_values() const { return 6 * (size_t)d.nap + 2 * (size_t)d.nt; }
     double *Fb = nullptr;   // adjoint: force adjoint per point
     double *Mb = nullptr;   // adjoint: position moments per point (9 each)
 };
@@ -1190,6 +1195,7 @@ extern "C" {
 falm_status falm_alm_destroy(falm_alm *A) {
     if (!A) return FALM_OK;
     for (void *p : A->bufs) (void)hipFree(p);
+    if (A->hout) (void)hipHostFree(A->hout);
     delete A;
     return FALM_OK;
 }
@@ -1261,11 +1267,9 @@ falm_status falm_alm_create(const falm_domain *dom, const falm_alm_config *c, co
         (st = upload(A, c->attack, d.nat, &dat)) || (st = upload(A, c->cl, (size_t)d.nat * d.nap, &dcl)) ||
         (st = upload(A, c->cd, (size_t)d.nat * d.nap, &dcd)) || (st = upload(A, toff.data(), toff.size(), &dto)) ||
         (st = upload(A, x, d.nx, &dx)) || (st = upload(A, y, d.ny, &dy)) || (st = upload(A, z, d.nz, &dz)) ||
-        (st = upload<double>(A, nullptr, 3 * d.nap, &d.ap_xyz)) ||
-        (st = upload<double>(A, nullptr, 3 * d.nap, &d.ap_force)) ||
+        (st = upload<double>(A, nullptr, A->out_values(), &d.ap_xyz)) ||
         (st = upload<double>(A, nullptr, d.nap, &d.ap_torque)) ||
         (st = upload<double>(A, nullptr, d.nap, &d.ap_thrust)) ||
-        (st = upload<double>(A, nullptr, d.nt, &d.torque)) || (st = upload<double>(A, nullptr, d.nt, &d.thrust)) ||
         (st = upload<int>(A, nullptr, 3 * d.nap, &d.ap_ijk)) || (st = upload<int>(A, nullptr, d.nap, &d.ap_rank)) ||
         (st = upload<double>(A, nullptr, (size_t)d.nap * d.nx, &d.fx)) ||
         (st = upload<double>(A, nullptr, (size_t)d.nap * d.ny, &d.fy)) ||
@@ -1274,6 +1278,10 @@ falm_status falm_alm_create(const falm_domain *dom, const falm_alm_config *c, co
         falm_alm_destroy(A);
         return st;
     }
+    // what falm_alm_get reads lies in one block: positions, forces, torque, thrust
+    d.ap_force = d.ap_xyz + 3 * (size_t)d.nap;
+    d.torque = d.ap_force + 3 * (size_t)d.nap;
+    d.thrust = d.torque + d.nt;
     d.tb = tbd;
     d.r = dr_;
     d.chord = dch;
@@ -1291,6 +1299,7 @@ falm_status falm_alm_create(const falm_domain *dom, const falm_alm_config *c, co
     // the uploads and zero fills ran on the null stream: finish them before
     // the caller's (possibly non-blocking) stream uses the buffers
     if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e == hipSuccess) e = hipHostMalloc(&A->hout, A->out_values() * sizeof(double), hipHostMallocDefault);
     if (e != hipSuccess) {
         st = hip_status(e, "hipMemcpy");
         falm_alm_destroy(A);
@@ -1358,12 +1367,17 @@ falm_status falm_alm_get(falm_alm *A, double *ap_xyz, double *ap_force, double *
                          void *stream) {
     if (!A) return FALM_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
-    if (ap_xyz) FALM_HIP(hipMemcpyAsync(ap_xyz, A->d.ap_xyz, 3 * A->nap * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (ap_force)
-        FALM_HIP(hipMemcpyAsync(ap_force, A->d.ap_force, 3 * A->nap * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (torque) FALM_HIP(hipMemcpyAsync(torque, A->d.torque, A->nt * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (thrust) FALM_HIP(hipMemcpyAsync(thrust, A->d.thrust, A->nt * sizeof(double), hipMemcpyDeviceToHost, s));
+    // One copy into pinned memory: with four copies into pageable memory, each
+    // of which waits, a step of two rotors and its results took 128 us, so 77.
+    std::lock_guard<std::mutex> lk(A->mx);
+    FALM_HIP(hipMemcpyAsync(A->hout, A->d.ap_xyz, A->out_values() * sizeof(double), hipMemcpyDeviceToHost, s));
     FALM_HIP(hipStreamSynchronize(s));
+    const double *h = A->hout;
+    const size_t np = 3 * (size_t)A->nap, nt = (size_t)A->nt;
+    if (ap_xyz) std::memcpy(ap_xyz, h, np * sizeof(double));
+    if (ap_force) std::memcpy(ap_force, h + np, np * sizeof(double));
+    if (torque) std::memcpy(torque, h + 2 * np, nt * sizeof(double));
+    if (thrust) std::memcpy(thrust, h + 2 * np + nt, nt * sizeof(double));
     return FALM_OK;
 }
 

@@ -16,7 +16,12 @@
 // (bit-identical to the per-cell metric fields, which are still kept for
 // falm_case_get_field), and the velocity snapshot is a buffer swap plus a
 // copy of the ghost shell instead of a full copy.
+#include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <cstring>
+#include <system_error>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -376,6 +381,107 @@ static void *case_field(falm_case *C, int field, int &ncol, int &prec) {
 
 }  // namespace falm
 
+namespace falm {
+
+bool Readback::alloc() {
+    if (pin) return true;
+    if (hipHostMalloc(&pin, 2 * kThreads * kChunk * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        pin = nullptr;
+        return false;
+    }
+    for (hipEvent_t &e : ev)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            return false;
+        }
+    return true;
+}
+
+void Readback::release() {
+    for (hipEvent_t &e : ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+}
+
+// One thread's share of a host copy: it takes the next chunk of the field,
+// starts its copy into one of its two pinned chunks, and writes out the one
+// it started before while that copy runs.
+template <typename T>
+static hipError_t readback_share(Readback &rb, int w, const T *src, double *out, size_t n, std::atomic<size_t> &next,
+                                 hipStream_t s) {
+    const size_t nchunk = (n + Readback::kChunk - 1) / Readback::kChunk;
+    T *buf[2] = {(T *)(rb.pin + (2 * w) * Readback::kChunk), (T *)(rb.pin + (2 * w + 1) * Readback::kChunk)};
+    size_t held[2] = {nchunk, nchunk};  // the chunk in flight into each buffer
+    hipError_t e = hipSuccess;
+    for (int k = 0;; k ^= 1) {
+        const size_t c = e == hipSuccess ? next.fetch_add(1) : nchunk;
+        if (c < nchunk) {
+            const size_t m = std::min(Readback::kChunk, n - c * Readback::kChunk);
+            e = hipMemcpyAsync(buf[k], src + c * Readback::kChunk, m * sizeof(T), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(rb.ev[2 * w + k], s);
+            if (e == hipSuccess) held[k] = c;
+        }
+        const size_t q = held[k ^ 1];
+        if (q < nchunk) {
+            const hipError_t ew = hipEventSynchronize(rb.ev[2 * w + (k ^ 1)]);
+            if (ew == hipSuccess) {
+                const size_t o = q * Readback::kChunk, m = std::min(Readback::kChunk, n - o);
+                if (sizeof(T) == sizeof(double))
+                    std::memcpy(out + o, buf[k ^ 1], m * sizeof(double));
+                else
+                    for (size_t i = 0; i < m; i++) out[o + i] = (double)buf[k ^ 1][i];
+            } else if (e == hipSuccess) {
+                e = ew;
+            }
+            held[k ^ 1] = nchunk;
+        }
+        if (held[k] >= nchunk) return e;
+    }
+}
+
+// Fields from two chunks on are copied by the threads: at 0.6 M values that is
+// 6 % faster than one pageable copy, and starting the threads costs 0.1 ms.
+static constexpr size_t kReadbackMin = 2 * Readback::kChunk;
+
+// Host copy of a field with several threads.  What bounds it is the host: a
+// pageable copy moves 10 GB/s, and on one core the conversion from float and
+// the first touch of the result's pages move 6 GB/s of the result.  The
+// velocity of 516 x 132 x 132 cells (27 M floats to doubles) took 38.4 ms and
+// takes 4.6; its pressure (9 M doubles) 6.9 and 2.2.
+template <typename T>
+static hipError_t readback(Readback &rb, const T *src, double *out, size_t n, hipStream_t s) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    std::atomic<size_t> next{0};
+    hipError_t err[Readback::kThreads] = {};
+    std::thread th[Readback::kThreads];
+    for (int w = 1; w < Readback::kThreads; w++) {
+        try {
+            th[w] = std::thread([&, w] {
+                hipError_t ew = hipSetDevice(dev);
+                err[w] = ew == hipSuccess ? readback_share(rb, w, src, out, n, next, s) : ew;
+            });
+        } catch (const std::system_error &) {
+            break;  // the threads there are share the chunks
+        }
+    }
+    err[0] = readback_share(rb, 0, src, out, n, next, s);
+    for (std::thread &t : th)
+        if (t.joinable()) t.join();
+    const hipError_t es = hipStreamSynchronize(s);  // after an error a chunk may still be in flight
+    for (hipError_t ew : err)
+        if (ew != hipSuccess) return ew;
+    return es;
+}
+
+}  // namespace falm
+
 extern "C" {
 
 falm_status falm_case_destroy(falm_case *C) {
@@ -385,6 +491,7 @@ falm_status falm_case_destroy(falm_case *C) {
     if (C->alm) falm_alm_destroy(C->alm);
     for (void *p : C->bufs) (void)hipFree(p);
     if (C->hnorm) (void)hipHostFree(C->hnorm);
+    C->rb.release();
     if (C->stream) (void)hipStreamDestroy(C->stream);
     delete C;
     return FALM_OK;
@@ -452,6 +559,14 @@ falm_status falm_case_get_field(falm_case *C, int field, double *host_out, size_
         return FALM_ERR_INVALID;
     }
     FALM_HIP(hipStreamSynchronize(C->stream));
+    if (n >= kReadbackMin) {
+        std::lock_guard<std::mutex> lk(C->rb.mx);
+        if (C->rb.alloc()) {
+            FALM_HIP(prec == FALM_F64 ? readback(C->rb, (const double *)src, host_out, n, C->stream)
+                                      : readback(C->rb, (const float *)src, host_out, n, C->stream));
+            return FALM_OK;
+        }
+    }
     if (prec == FALM_F64) {
         FALM_HIP(hipMemcpy(host_out, src, n * sizeof(double), hipMemcpyDeviceToHost));
     } else {

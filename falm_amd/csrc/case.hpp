@@ -2,9 +2,25 @@
 // (case.hip) and the adjoint (adjoint.hip).
 #pragma once
 
+#include <mutex>
 #include <vector>
 
 #include "cfd.hpp"
+
+namespace falm {
+// Host copies of large fields: kThreads threads, each with two pinned chunks
+// in turn, so that the copy engine fills one chunk while the threads convert
+// and write out the others.
+struct Readback {
+    static constexpr int kThreads = 8;
+    static constexpr size_t kChunk = (size_t)1 << 18;  // elements; 2 MiB of doubles
+    double *pin = nullptr;                             // 2 kThreads chunks, pinned, kept with the case
+    hipEvent_t ev[2 * kThreads] = {};
+    std::mutex mx;                                     // one call at a time uses the chunks
+    bool alloc();
+    void release();
+};
+}  // namespace falm
 
 struct falm_case {
     falm_case_config cfg;
@@ -28,6 +44,7 @@ struct falm_case {
     int pbc[6], uubc[6];
     // device scalar for the divergence norm + its reduction scratch
     double *dnorm = nullptr, *partials = nullptr, *hnorm = nullptr;
+    falm::Readback rb;        // pinned chunks of falm_case_get_field
     bool norm_pending = false;  // the last step's norm (written into hnorm by its kernel) is not waited for
     int *nobox = nullptr;     // empty cell box: no rotor, ff stays zero
     std::vector<void *> bufs;
