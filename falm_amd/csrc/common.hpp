@@ -234,8 +234,7 @@ inline dim3 ew_grid(size_t n) {
 // permutes a step, 12 a sum, and the waves of a reduction share one LDS.
 // With the values of a block side by side on its waves (block_sum_n) the
 // finalize and the ends of the reducing kernels got shorter: the window
-// gradient at 96 x 48 x 48 64.1 -> 59.8 ms, the cavity solve at 128^3 960 ->
-// 943 us.  Every lane gets the sum; all 64 must be active.
+// gradient at 96 x 48 x 48 64.1 -> 59.8 ms.  Every lane gets the sum; all 64 must be active.
 template <int CTRL, int ROWS>
 __device__ inline double dpp_shifted(double v) {  // 0 where a lane receives none
     const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);

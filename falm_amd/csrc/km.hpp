@@ -35,9 +35,7 @@ struct K7Tiling {
 // CUs (pseudo-velocity 30 us, 17 us Smagorinsky and divergence).  The line
 // lies at two workgroups a CU: on MI355X the wind-tunnel step in double took
 // 660 us at 64 x 33 x 30 with 16 planes a chunk, 416 us filled to 256
-// workgroups and 400 us to 512; at 128^3 cells two k_sor3_km workgroups fit a
-// CU (LDS), and the cavity solve took 1109 us unfilled, 960 us at 512 and
-// 1075 us at 1024.
+// workgroups and 400 us to 512.
 #ifndef FALM_K7_KC
 #define FALM_K7_KC 16
 #endif

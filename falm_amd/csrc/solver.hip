@@ -778,218 +778,287 @@ __global__ __launch_bounds__(K7_NT) __attribute__((amdgpu_waves_per_eu(PcmvWaves
 }
 
 // ---------------------------------------------------------------------
-// Three red-black SOR half-sweeps (colours c0, 1-c0, c0) in one pass over
-// memory, out of place (x_in -> x_out).  A workgroup owns an S3_BX x S3_BY
-// column of cells and marches its planes in k with the three sweeps skewed:
-// while plane s gets sweep 1, plane s-1 gets sweep 2 and plane s-2 sweep 3,
-// each in LDS.  A cell's update reads its six neighbours, which have the
-// other colour, so sweep 2 at plane s-1 needs sweep-1 values on planes
-// s-2..s and sweep 3 at s-2 needs sweep-2 values on s-3..s-1: the skew gives
-// both.  In x and y the sweeps are computed redundantly on rings of the
-// tile (sweep 1 on the tile plus 2 cells, sweep 2 plus 1, sweep 3 on the
-// tile), from the same input values a neighbouring workgroup uses, so the
-// written cells equal those of three separate sweeps bit for bit.  The same
-// holds in k across the chunk ends.  Per cell this reads x, b and the
-// diagonal once and writes x once, where three separate half-sweeps read
-// and write x three times.
-constexpr int S3_BX = 64, S3_BY = 8, S3_NT = S3_BX * S3_BY;
-constexpr int S3_R = 3;                     // x ring (sweep 1 on ring 2 reads ring 3)
-constexpr int S3_W = S3_BX + 2 * S3_R, S3_H = S3_BY + 2 * S3_R;
-constexpr int S3_PL = S3_W * S3_H;          // x cells per plane
-constexpr int S3_NXP = 5;                   // x planes in flight: s+2 .. s-2
-constexpr int S3_RB = 2;                    // b / diagonal ring
-constexpr int S3_BW = S3_BX + 2 * S3_RB, S3_BH = S3_BY + 2 * S3_RB;
-constexpr int S3_BPL = S3_BW * S3_BH;       // b cells per plane
-constexpr int S3_NBP = 3;                   // b planes in flight: s+1 .. s-1
-constexpr int S3_KC = 16;                   // output planes per chunk at most
-constexpr int S3_XPT = (S3_PL + S3_NT - 1) / S3_NT;   // x cells per thread per plane
-constexpr int S3_BPT = (S3_BPL + S3_NT - 1) / S3_NT;  // b cells per thread per plane
+// The preconditioner with two red-black sweeps from x = 0 (half-sweeps B1,
+// R1, B2, R2) and the operator product on its result, in one pass over
+// memory: pc = M(v), out = A M(v), with the dot products of
+// kernel_PBiCGStab's steps.
+//
+// What bounds the work is arithmetic: two divisions and three seven-term sums
+// a cell in FP64.  A thread owns P2_C columns, consecutive in y, of a region
+// of 64 x P2_RY columns and marches them in k with the half-sweeps skewed two
+// planes apart, so that one barrier a step is enough: step s forms B1 on
+// plane s+2, R1 on s, B2 on s-2, R2 on s-4 and A on s-5.  The region holds
+// the tile and four rings around it, on which the half-sweeps are repeated
+// (each half-sweep needs one ring less than the one before), from the same
+// values that a neighbouring workgroup uses.
+//
+// A cell's colour is that of the cells two planes away, so in a step a lane
+// is either black at s (it does B1 and B2) or red (R1 and R2): each lane
+// divides twice a step and none idles on the other colour.  `first` below is
+// B1 or R1 (plane s+2 or s), `second` B2 or R2, always four planes below the
+// first, so what the first used (v, the diagonal) the second takes from
+// registers four steps later.  The last four steps' values of both are kept,
+// indexed by step; with x(s) a column's value in step s, the neighbours are
+//   first,  red:   k+-1: own first(s-1), first(s-3); x, y: first(s-2)
+//   second, black: k+-1: own first(s-1), first(s-3); x, y: first(s-2)
+//   second, red:   k+-1: own second(s-1), second(s-3); x, y: second(s-2)
+//   A's plane s-5: second(s-1) where black at s, else second(s-3)
+// x neighbours are lane shifts (the wave is a row of the region), y
+// neighbours the thread's own other column or, through LDS, the next wave's.
+// Cells outside the interior hold zero, as the ghost
+// cells of the preconditioned vectors do.
+//
+// At 128^3 cells in double a launch takes 39 us where the three half-sweeps
+// (B1 was in the p and s kernels) and the operator product took 36 + 13.5 and
+// the p and s kernels 4.5 more each; the vector unit issues half the time.
+// The cavity solve (6 iterations) 943 -> 795 us, in mixed precision 832 ->
+// 622; 512 x 128 x 128 in double 2400 -> 1888, mixed 1458 -> 1217; 40^3 1618
+// -> 646.  Tried in double: 4 columns a thread on 8 waves 832 us (256 VGPRs,
+// two waves a SIMD; with the sums kept unconditional it spills), 4 waves 919,
+// 2 columns on 8 waves 911, 10 waves 838, 11 waves 827, 16 waves 1174 (spills
+// at 128 VGPRs).
+constexpr int P2_C = 2, P2_NW = 12, P2_NT = 64 * P2_NW;
+constexpr int P2_RY = P2_C * P2_NW;         // region rows
+constexpr int P2_R = 4;                     // rings
+constexpr int P2_OX = 64 - 2 * P2_R, P2_OY = P2_RY - 2 * P2_R;  // tile
 
-struct S3Tiling {
+struct P2Tiling {
     Box box;  // the interior
     int tx, ty, tk;
-    int kc;  // output planes per chunk
+    int kc;  // planes per chunk
     int blocks;
 };
-inline S3Tiling make_s3_tiling(const Box &b) {
-    S3Tiling t;
+// Tiles along an axis of n cells: the first and the last region need no ring
+// at the domain's end.
+inline int p2_tiles(int n, int region) {
+    if (n <= region) return 1;
+    const int rest = n - 2 * (region - P2_R), o = region - 2 * P2_R;
+    return 2 + (rest > 0 ? (rest + o - 1) / o : 0);
+}
+// One double workgroup runs on a CU (162 VGPRs, 115 KB of LDS), so the time is the rounds of 256
+// workgroups times a chunk's steps; a chunk of n planes takes n + 11, of which
+// the first six and the last two do one half-sweep pair of the two.
+inline P2Tiling make_p2_tiling(const Box &b) {
+    P2Tiling t;
     t.box = b;
-    t.tx = (b.n[0] + S3_BX - 1) / S3_BX;
-    t.ty = (b.n[1] + S3_BY - 1) / S3_BY;
-    t.kc = k7_chunk(t.tx * t.ty, b.n[2], S3_KC);
-    t.tk = (b.n[2] + t.kc - 1) / t.kc;
-    t.blocks = (b.n[0] > 0 && b.n[1] > 0 && b.n[2] > 0) ? t.tx * t.ty * t.tk : 0;
+    t.tx = p2_tiles(b.n[0], 64);
+    t.ty = p2_tiles(b.n[1], P2_RY);
+    t.kc = 1;
+    t.tk = t.blocks = 0;
+    if (b.n[0] <= 0 || b.n[1] <= 0 || b.n[2] <= 0) return t;
+    const long cols = (long)t.tx * t.ty;
+    long best = LONG_MAX;
+    for (int kc = 1; kc <= b.n[2]; kc++) {
+        const long tk = (b.n[2] + kc - 1) / kc;
+        if (cols * tk > RED_BLOCKS) continue;
+        const long cost = ((cols * tk + 255) / 256) * (kc + 7);
+        if (cost >= best) continue;
+        best = cost;
+        t.kc = kc;
+        t.tk = (int)tk;
+        t.blocks = (int)(cols * tk);
+    }
     return t;
 }
 
-template <class T>
-__global__ __launch_bounds__(S3_NT) void k_sor3_km(S3Tiling kt, Geom g, OpSep<T> a, const T *__restrict__ xin,
-                                                   T *__restrict__ xout, const T *__restrict__ b, T omega, int c0,
-                                                   const int *done) {
-    if (*done) return;
-    __shared__ T sx[S3_NXP][S3_PL];
-    __shared__ T sb[S3_NBP][S3_BPL], sd[S3_NBP][S3_BPL];
-    __shared__ T saw[S3_W], sae[S3_W], sas[S3_H], san[S3_H];
+// a row's values one lane along, zero at its end
+template <int CTRL>
+__device__ inline double p2_shift(double v) { return dpp_shifted<CTRL, 0xf>(v); }
+template <int CTRL>
+__device__ inline float p2_shift(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// x is computed in every lane: without this the compiler branches around sums
+// and divisions whose result a select or a store drops, and those of a
+// thread's columns no longer overlap (824 us for 795)
+__device__ inline void p2_keep(double &x) { asm("" : "+v"(x)); }
+__device__ inline void p2_keep(float &x) { asm("" : "+v"(x)); }
+
+// MODE 1: w is rr, partials (rr, out); MODE 2: w is v, partials (out, v),
+// (out, out)
+template <class T, int MODE>
+__global__ __launch_bounds__(P2_NT) __attribute__((amdgpu_waves_per_eu(P2_NW / 4))) void k_bicg_pc2mv_km(
+    P2Tiling kt, Geom g, OpSep<T> a, const T *__restrict__ v, const T *__restrict__ w, T *__restrict__ pc,
+    T *__restrict__ out, const DevState *st, T omega_pc, double *partials) {
+    if (st->done) return;
+    constexpr int C = P2_C;
+    // [step & 3][first, second][wave + 1][its first, last column][lane]; the
+    // planes of waves -1 and P2_NW stay zero
+    __shared__ T pub[4][2][P2_NW + 2][2][64];
+    __shared__ double lds[2 * P2_NW];
     const int L = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x));
     const int bx = L % kt.tx, by = (L / kt.tx) % kt.ty, kc = L / (kt.tx * kt.ty);
-    const int i0 = kt.box.lo[0] + bx * S3_BX, j0 = kt.box.lo[1] + by * S3_BY;
-    const int ilo = kt.box.lo[0], ihi = kt.box.lo[0] + kt.box.n[0];  // interior [lo, hi)
-    const int jlo = kt.box.lo[1], jhi = kt.box.lo[1] + kt.box.n[1];
-    const int klo = kt.box.lo[2], khi = kt.box.lo[2] + kt.box.n[2];
-    const int k0 = klo + kc * kt.kc, k1 = min(k0 + kt.kc, khi);  // output planes
-    const int t = (int)threadIdx.x;
-    const int sz = g.nxy;
-    // 1-D operator coefficients of the tile's x and y range
-    for (int q = t; q < S3_W + S3_H; q += S3_NT) {
-        if (q < S3_W) {
-            const int gi = min(max(i0 - S3_R + q, 0), g.nx - 1);
-            saw[q] = a.aw[gi];
-            sae[q] = a.ae[gi];
-        } else {
-            const int gj = min(max(j0 - S3_R + (q - S3_W), 0), g.ny - 1);
-            sas[q - S3_W] = a.as[gj];
-            san[q - S3_W] = a.an[gj];
-        }
+    const int lo0 = kt.box.lo[0], hi0 = lo0 + kt.box.n[0], lo1 = kt.box.lo[1], hi1 = lo1 + kt.box.n[1];
+    const int lo2 = kt.box.lo[2], hi2 = lo2 + kt.box.n[2];
+    const int k0 = lo2 + kc * kt.kc, k1 = min(k0 + kt.kc, hi2);
+    const int lane = (int)(threadIdx.x & 63), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int i = lo0 + P2_OX * bx + lane, j0 = lo1 + P2_OY * by + C * wv;
+    const bool inx = i < hi0;
+    const int ii = inx ? i : hi0 - 1;  // a column outside the interior loads a valid one
+    const bool ox = inx && (bx == 0 || lane >= P2_R) && (bx == kt.tx - 1 || lane < 64 - P2_R);
+    const T ae = a.ae[ii], aw = a.aw[ii];
+    T an[C], as[C];
+    unsigned cb[C];
+    bool in[C], wr[C];
+#pragma unroll
+    for (int r = 0; r < C; r++) {
+        const int jj = min(j0 + r, hi1 - 1), jr = C * wv + r;
+        an[r] = ld_uniform(a.an, jj);
+        as[r] = ld_uniform(a.as, jj);
+        cb[r] = (unsigned)(ii + g.nx * jj) * sizeof(T);
+        in[r] = inx && j0 + r < hi1;
+        wr[r] = ox && j0 + r < hi1 && (by == 0 || jr >= P2_R) && (by == kt.ty - 1 || jr < P2_RY - P2_R);
     }
-    // this thread's load slots: x on ring 3, b and the diagonal on ring 2
-    // (cells outside the array load nothing; no update reads them)
-    unsigned xo[S3_XPT], bo[S3_BPT];
-    bool xok[S3_XPT], bok[S3_BPT];
-#pragma unroll
-    for (int q = 0; q < S3_XPT; q++) {
-        const int c = t + q * S3_NT;
-        const int gi = i0 - S3_R + c % S3_W, gj = j0 - S3_R + c / S3_W;
-        xok[q] = c < S3_PL && gi >= 0 && gi < g.nx && gj >= 0 && gj < g.ny;
-        xo[q] = xok[q] ? (unsigned)(gi + g.nx * gj) * sizeof(T) : 0u;
+    const unsigned szt = (unsigned)g.nxy * sizeof(T);
+    const auto kin = [&](int k) { return k >= lo2 && k < hi2; };
+    const auto kcl = [&](int k) { return k < lo2 ? lo2 : (k >= hi2 ? hi2 - 1 : k); };
+    for (int q = (int)threadIdx.x; q < 4 * 2 * 2 * 64; q += P2_NT) {
+        const int l = q & 63, c = (q >> 6) & 1, f = (q >> 7) & 1, s = q >> 8;
+        pub[s][f][0][c][l] = T(0);
+        pub[s][f][P2_NW + 1][c][l] = T(0);
     }
+    // s0: the first step; blk0: column 0's cell is black at plane s0
+    const int s0 = k0 - 6;
+    const bool blk0 = ((i + j0 + s0 + g.osum) & 1) == FALM_COLOR_BLACK;
+    T X1[C][4], X2[C][4], V[C][4], D[C][4], nv[C], nd[C], nw[C], na[C];
 #pragma unroll
-    for (int q = 0; q < S3_BPT; q++) {
-        const int c = t + q * S3_NT;
-        const int gi = i0 - S3_RB + c % S3_BW, gj = j0 - S3_RB + c / S3_BW;
-        bok[q] = c < S3_BPL && gi >= 0 && gi < g.nx && gj >= 0 && gj < g.ny;
-        bo[q] = bok[q] ? (unsigned)(gi + g.nx * gj) * sizeof(T) : 0u;
+    for (int r = 0; r < C; r++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) X1[r][q] = X2[r][q] = V[r][q] = T(0), D[r][q] = T(1);
+        nw[r] = T(0);
+        na[r] = T(1);
     }
-    const unsigned szb = (unsigned)sz * sizeof(T);
-    auto load_x = [&](int k, T (&v)[S3_XPT]) {
-        const bool kin = k >= 0 && k < g.nz;
+    // v and the diagonal of step s's first half-sweeps; b0: column 0 is black
+    const auto fetch = [&](int s, bool b0) {
+        const unsigned ob = (unsigned)kcl(s + 2) * szt, orr = (unsigned)kcl(s) * szt;
+        const unsigned oe = b0 ? ob : orr, oo = b0 ? orr : ob;
 #pragma unroll
-        for (int q = 0; q < S3_XPT; q++) v[q] = (kin && xok[q]) ? ld_at(xin, xo[q] + (unsigned)k * szb) : T(0);
-    };
-    auto load_b = [&](int k, T (&vb)[S3_BPT], T (&vd)[S3_BPT]) {
-        const bool kin = k >= 0 && k < g.nz;
-#pragma unroll
-        for (int q = 0; q < S3_BPT; q++) {
-            const bool ok = kin && bok[q];
-            vb[q] = ok ? ld_at(b, bo[q] + (unsigned)k * szb) : T(0);
-            vd[q] = ok ? ld_at(a.ac, bo[q] + (unsigned)k * szb) : T(1);
-        }
-    };
-    auto store_x = [&](int k, const T (&v)[S3_XPT]) {
-        T *p = sx[((k % S3_NXP) + S3_NXP) % S3_NXP];
-#pragma unroll
-        for (int q = 0; q < S3_XPT; q++)
-            if (t + q * S3_NT < S3_PL) p[t + q * S3_NT] = v[q];
-    };
-    auto store_b = [&](int k, const T (&vb)[S3_BPT], const T (&vd)[S3_BPT]) {
-        const int sl = ((k % S3_NBP) + S3_NBP) % S3_NBP;
-#pragma unroll
-        for (int q = 0; q < S3_BPT; q++)
-            if (t + q * S3_NT < S3_BPL) {
-                sb[sl][t + q * S3_NT] = vb[q];
-                sd[sl][t + q * S3_NT] = vd[q];
-            }
-    };
-    // one SOR update of x-buffer cell (xi, yi) of plane k (colour already
-    // checked by the caller): k_sor_op's expression
-    auto update = [&](int k, int xi, int yi, T atk, T abk) {
-        T *xc_p = sx[k % S3_NXP];
-        const T *xm = sx[(k + S3_NXP - 1) % S3_NXP], *xp = sx[(k + 1) % S3_NXP];
-        const int c = xi + S3_W * yi;
-        const int sl = k % S3_NBP, cbi = (xi - (S3_R - S3_RB)) + S3_BW * (yi - (S3_R - S3_RB));
-        const T xc = xc_p[c];
-        const T ac = sd[sl][cbi];
-        const T s = ac * xc + sae[xi] * xc_p[c + 1] + saw[xi] * xc_p[c - 1] + san[yi] * xc_p[c + S3_W] +
-                    sas[yi] * xc_p[c - S3_W] + atk * xp[c] + abk * xm[c];
-        const T cv = (sb[sl][cbi] - s) / ac;
-        xc_p[c] = xc + omega * cv;
-    };
-    // sweep with colour col on ring r of plane k, interior cells only.  A
-    // ring row of even width holds w/2 cells of each colour: thread c takes
-    // the c-th cell of the colour, so no lane idles on the other colour.
-    auto sweep = [&](int k, int r, int col) {
-        if (k < klo || k >= khi) return;  // uniform: ghost planes are not updated
-        const int w = S3_BX + 2 * r, h = S3_BY + 2 * r, half = w / 2;
-        const int gi0 = i0 - r;
-        const T atk = a.at[k], abk = a.ab[k];  // before the loop: one wait for both
-        for (int c = t; c < half * h; c += S3_NT) {
-            const int yr = c / half, xr = 2 * (c - yr * half);
-            const int gj = j0 - r + yr;
-            const int gi = gi0 + xr + ((col - gi0 - gj - k - g.osum) & 1);
-            if (gi < ilo || gi >= ihi || gj < jlo || gj >= jhi) continue;
-            update(k, gi - (i0 - S3_R), gj - (j0 - S3_R), atk, abk);
+        for (int r = 0; r < C; r++) {
+            const unsigned o = cb[r] + ((r & 1) ? oo : oe);
+            nv[r] = ld_at(v, o);
+            nd[r] = ld_at(a.ac, o);
         }
     };
-    // Sweep 3 works per column: thread t owns column (i0 + t % BX, j0 + t / BX)
-    // and keeps its final value of the previous plane, b and the diagonal
-    // of its cell in registers, so neither plane s-3 nor b of plane s-2
-    // occupies LDS.
-    const int oi = i0 + t % S3_BX, oj = j0 + t / S3_BX;
-    const bool own = oi < ihi && oj < jhi;
-    const int oxi = oi - (i0 - S3_R), oyi = oj - (j0 - S3_R);
-    const unsigned oo = own ? (unsigned)(oi + g.nx * oj) * sizeof(T) : 0u;
-    T xprev = T(0), ob = T(0), od = T(1), nb_ = T(0), nd_ = T(1);
-    auto load_own = [&](int k, T &vb_, T &vd_) {
-        if (own && k >= klo && k < khi) {
-            vb_ = ld_at(b, oo + (unsigned)k * szb);
-            vd_ = ld_at(a.ac, oo + (unsigned)k * szb);
-        }
-    };
-    // prologue: x planes k0-3 .. k0-1 and b plane k0-2 in LDS, x plane k0
-    // and b plane k0-1 in registers
-    T vx[S3_XPT], vb[S3_BPT], vd[S3_BPT];
-    for (int k = k0 - 3; k < k0; k++) {
-        load_x(k, vx);
-        store_x(k, vx);
-    }
-    load_b(k0 - 2, vb, vd);
-    store_b(k0 - 2, vb, vd);
-    load_x(k0, vx);
-    load_b(k0 - 1, vb, vd);
+    // the operator's k coefficients on planes s, s-1 .. s-5
+    T at[6], ab[6];
+#pragma unroll
+    for (int m = 0; m < 6; m++) at[m] = ld_uniform(a.at, kcl(s0 - m)), ab[m] = ld_uniform(a.ab, kcl(s0 - m));
+    fetch(s0, blk0);
+    double acc[2] = {0.0, 0.0};
     __syncthreads();
-    const int c1 = 1 - c0;
-    // Iteration s: sweep 1 on plane s, sweep 2 on s-1, sweep 3 on s-2.  The
-    // LDS slots written at the top of the iteration (x plane s+2, b plane
-    // s+1) were last read during iteration s-1, before its final barrier.
-    for (int s = k0 - 2; s < k1 + 2; s++) {
-        if (s + 2 <= k1 + 2) store_x(s + 2, vx);
-        if (s + 1 <= k1 + 1) store_b(s + 1, vb, vd);
-        if (s + 3 <= k1 + 2) load_x(s + 3, vx);
-        if (s + 2 <= k1 + 1) load_b(s + 2, vb, vd);
-        ob = nb_;
-        od = nd_;
-        load_own(s - 1, nb_, nd_);  // the own cell of the next sweep-3 plane
-        sweep(s, 2, c0);
-        __syncthreads();
-        if (s - 1 >= k0 - 1) sweep(s - 1, 1, c1);
-        __syncthreads();
-        const int k = s - 2;
-        if (k == k0 - 1 && own) xprev = sx[k % S3_NXP][oxi + S3_W * oyi];  // final below the chunk
-        if (k >= k0 && own) {
-            // sweep 3 on the own column's cell: its k-1 neighbour is the
-            // final value kept from the previous plane
-            T *xc_p = sx[k % S3_NXP];
-            const int c = oxi + S3_W * oyi;
-            T v = xc_p[c];
-            if (((oi + oj + k + g.osum) & 1) == c0) {
-                const T sr = od * v + sae[oxi] * xc_p[c + 1] + saw[oxi] * xc_p[c - 1] + san[oyi] * xc_p[c + S3_W] +
-                             sas[oyi] * xc_p[c - S3_W] + a.at[k] * sx[(k + 1) % S3_NXP][c] + a.ab[k] * xprev;
-                const T cv = (ob - sr) / od;
-                v = v + omega * cv;
+    const auto step = [&](int s, auto qc) {
+        constexpr int q = decltype(qc)::value, m1 = (q + 3) & 3, m2 = (q + 2) & 3, m3 = (q + 1) & 3;
+        const bool b0 = (q & 1) ? !blk0 : blk0;
+        T x1[C], v1[C], d1[C];
+#pragma unroll
+        for (int r = 0; r < C; r++) v1[r] = nv[r], d1[r] = nd[r], x1[r] = T(0);
+        // the rows beyond the thread's own: j+1 of its last, j-1 of its first
+        const T u1 = pub[m2][0][wv + 2][0][lane], u2 = pub[m2][1][wv + 2][0][lane];
+        const T l1 = pub[m2][0][wv][1][lane], l2 = pub[m2][1][wv][1][lane];
+        static_assert(C % 2 == 0, "the last column has the colour opposite to the first");
+        const T uc = pub[b0 ? m1 : m3][1][wv + 2][0][lane];  // the last column is red where the first is black
+        const T lc = pub[b0 ? m3 : m1][1][wv][1][lane];
+        const T atn = ld_uniform(a.at, kcl(s + 1)), abn = ld_uniform(a.ab, kcl(s + 1));
+        if (s < k1 + 2) fetch(s + 1, !b0);
+        // A's operands: loaded here, a step's arithmetic ahead, and not next
+        // to the stores of the step before, for which they would wait
+        const int k = s - 5;
+        if (k >= k0) {
+#pragma unroll
+            for (int r = 0; r < C; r++) {
+                const unsigned ob = cb[r] + (unsigned)k * szt;
+                nw[r] = ld_at(w, ob);
+                na[r] = ld_at(a.ac, ob);
             }
-            st_at(xout, oo + (unsigned)k * szb, v);
-            xprev = v;
         }
+        if (s <= k1 + 2) {
+            const bool kb = kin(s + 2), kr = kin(s);
+#pragma unroll
+            for (int r = 0; r < C; r++) {
+                const bool b = (r & 1) ? !b0 : b0;
+                const T xn = r + 1 < C ? X1[r + 1 < C ? r + 1 : r][m2] : u1, xs = r > 0 ? X1[r > 0 ? r - 1 : 0][m2] : l1;
+                T sum = ae * p2_shift<0x130>(X1[r][m2]) + aw * p2_shift<0x138>(X1[r][m2]) + an[r] * xn +
+                              as[r] * xs + at[0] * X1[r][m1] + ab[0] * X1[r][m3];
+                p2_keep(sum);
+                T x = T(0) + omega_pc * ((b ? v1[r] : v1[r] - sum) / d1[r]);
+                p2_keep(x);
+                x1[r] = in[r] && (b ? kb : kr) ? x : T(0);
+            }
+        }
+        if (s >= k0) {
+            const bool kb = kin(s - 2), kr = kin(s - 4);
+            T y[C], x2[C];
+#pragma unroll
+            for (int r = 0; r < C; r++) {
+                const bool b = (r & 1) ? !b0 : b0;
+                y[r] = b ? X2[r][m2] : X1[r][m2];
+            }
+#pragma unroll
+            for (int r = 0; r < C; r++) {
+                const bool b = (r & 1) ? !b0 : b0;
+                // beyond the thread's rows the neighbour has the other colour
+                const T xn = r + 1 < C ? y[r + 1 < C ? r + 1 : r] : (b ? u1 : u2);
+                const T xs = r > 0 ? y[r > 0 ? r - 1 : 0] : (b ? l1 : l2);
+                const T xc = X1[r][q];
+                const T sum = D[r][q] * xc + ae * p2_shift<0x130>(y[r]) + aw * p2_shift<0x138>(y[r]) + an[r] * xn +
+                              as[r] * xs + (b ? at[2] : at[4]) * (b ? X1[r][m1] : X2[r][m1]) +
+                              (b ? ab[2] : ab[4]) * (b ? X1[r][m3] : X2[r][m3]);
+                T x = xc + omega_pc * ((V[r][q] - sum) / D[r][q]);
+                p2_keep(x);
+                x2[r] = in[r] && (b ? kb : kr) ? x : T(0);
+            }
+            if (k >= k0) {
+                T c[C];
+#pragma unroll
+                for (int r = 0; r < C; r++) c[r] = ((r & 1) ? !b0 : b0) ? X2[r][m1] : X2[r][m3];
+#pragma unroll
+                for (int r = 0; r < C; r++) {
+                    const bool b = (r & 1) ? !b0 : b0;
+                    const T xn = r + 1 < C ? c[r + 1 < C ? r + 1 : r] : uc, xs = r > 0 ? c[r > 0 ? r - 1 : 0] : lc;
+                    T o = na[r] * c[r] + ae * p2_shift<0x130>(c[r]) + aw * p2_shift<0x138>(c[r]) + an[r] * xn +
+                                as[r] * xs + at[5] * (b ? X2[r][m2] : x2[r]) + ab[5] * (b ? X2[r][q] : X2[r][m2]);
+                    p2_keep(o);
+                    if (wr[r]) {
+                        const unsigned ob = cb[r] + (unsigned)k * szt;
+                        st_at(pc, ob, c[r]);
+                        st_at(out, ob, o);
+                        acc[0] += (double)nw[r] * (double)o;
+                        if (MODE == 2) acc[1] += (double)o * (double)o;
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < C; r++) X2[r][q] = x2[r];
+            pub[q][1][wv + 1][0][lane] = x2[0];
+            pub[q][1][wv + 1][1][lane] = x2[C - 1];
+        }
+#pragma unroll
+        for (int r = 0; r < C; r++) X1[r][q] = x1[r], V[r][q] = v1[r], D[r][q] = d1[r];
+#pragma unroll
+        for (int m = 5; m > 0; m--) at[m] = at[m - 1], ab[m] = ab[m - 1];
+        at[0] = atn;
+        ab[0] = abn;
+        pub[q][0][wv + 1][0][lane] = x1[0];
+        pub[q][0][wv + 1][1][lane] = x1[C - 1];
         __syncthreads();
+    };
+    using std::integral_constant;
+    for (int s = s0;; s += 4) {
+        step(s, integral_constant<int, 0>{});
+        if (s + 1 > k1 + 4) break;
+        step(s + 1, integral_constant<int, 1>{});
+        if (s + 2 > k1 + 4) break;
+        step(s + 2, integral_constant<int, 2>{});
+        if (s + 3 > k1 + 4) break;
+        step(s + 3, integral_constant<int, 3>{});
+        if (s + 4 > k1 + 4) break;
+    }
+    if (MODE == 1) {
+        double a1[1] = {acc[0]};
+        block_partials<P2_NT, 1>(a1, partials, lds);
+    } else {
+        block_partials<P2_NT, 2>(acc, partials, lds);
     }
 }
 
@@ -1108,7 +1177,7 @@ __global__ __launch_bounds__(FIN_NT) void k_fin_check(DevState *st, const double
 }
 
 // p = r (first) or r + beta(p - omega q) (kernel_PBiCGStab_1), then the
-// first preconditioner sweep pp = M0(p)
+// first preconditioner sweep pp = M0(p), unless a later kernel forms it (no pp)
 template <class T, class OP>
 __global__ __launch_bounds__(NT) void k_bicg_p(Tiling tl, Geom g, OP a, const T *__restrict__ r, T *__restrict__ p,
                                                const T *__restrict__ q, T *__restrict__ pp, const DevState *st,
@@ -1124,7 +1193,7 @@ __global__ __launch_bounds__(NT) void k_bicg_p(Tiling tl, Geom g, OP a, const T 
             pv = r[cc] + beta * (p[cc] - omega * q[cc]);
         }
         p[cc] = pv;
-        pp[cc] = pc_first<T>(pc_type, omega_pc, pv, a.diag(cc), ((i + j + k + g.osum) & 1) == FALM_COLOR_BLACK);
+        if (pp) pp[cc] = pc_first<T>(pc_type, omega_pc, pv, a.diag(cc), ((i + j + k + g.osum) & 1) == FALM_COLOR_BLACK);
     });
 }
 
@@ -1139,7 +1208,7 @@ __global__ __launch_bounds__(NT) void k_bicg_s(Tiling tl, Geom g, OP a, const T 
         const T alpha = (T)st->alpha;
         const T sv = r[cc] - alpha * q[cc];
         s[cc] = sv;
-        ss[cc] = pc_first<T>(pc_type, omega_pc, sv, a.diag(cc), ((i + j + k + g.osum) & 1) == FALM_COLOR_BLACK);
+        if (ss) ss[cc] = pc_first<T>(pc_type, omega_pc, sv, a.diag(cc), ((i + j + k + g.osum) & 1) == FALM_COLOR_BLACK);
     });
 }
 
@@ -1783,7 +1852,7 @@ struct falm_solver {
     Tiling tp;     // tiles of x-adjacent cell pairs (k_bicg_update2); no tiles when pairs are not aligned
     K7Tiling kt;   // k-marching column tiles of the interior (stencil kernels)
     K7Tiling ktp;  // the same for k_bicg_pcmv_km (its own chunk length)
-    S3Tiling s3;   // tiles of the fused three-sweep SOR kernel
+    P2Tiling p2;   // tiles of the two-sweep preconditioner with the operator product
     S2Tiling s2;   // tiles of the one-layer SOR solver
     DevState *st = nullptr;
     DevState *hst = nullptr;  // pinned mirror
@@ -1927,30 +1996,14 @@ static double diag_bytes(const falm_solver *S) {
 
 // preconditioner sweeps after the fused first one (SORPC: pc_maxit x
 // {black, red}; JacobiPC: pc_maxit sweeps; both run at least once,
-// src/FalmEq.cpp:147-170,258-302).  Returns the vector holding the result:
-// x itself, or `spare` when the three sweeps of pc_maxit = 2 on a separable
-// double operator run as one out-of-place pass (k_sor3_km).
+// src/FalmEq.cpp:147-170,258-302), in place.
 template <class T, class OP>
-static T *pc_rest(falm_solver *S, const OP &a, T *x, const T *b, T *spare, hipStream_t s, falm_status &st) {
+static falm_status pc_rest(falm_solver *S, const OP &a, T *x, const T *b, hipStream_t s) {
     const falm_solver_config &c = S->cfg;
     const int m = c.pc_maxit < 1 ? 1 : c.pc_maxit;
     const int *done = &S->st->done;
     const T w = (T)c.pc_relax;
-    st = FALM_OK;
     if (c.pc_type == FALM_LS_SOR) {
-        // the fused pass pays off in double (measured on MI355X at
-        // 512x128x128: 127 us against 3 x 58 us); in float the three
-        // separate half-sweeps (3 x 27 us) stay faster than its 80-95 us
-        if constexpr (std::is_same<T, double>::value && std::is_same<OP, OpSep<T>>::value) {
-            if (m == 2 && S->s3.blocks > 0) {
-                TimedLaunch tm(FALM_TIME_SOR, s);
-                hipLaunchKernelGGL((k_sor3_km<T>), dim3(S->s3.blocks), dim3(S3_NT), 0, s, S->s3, S->g, a,
-                                   (const T *)x, spare, b, w, FALM_COLOR_RED, done);
-                tm.done((double)S->tl.box.size() * 4.0 * sizeof(T));
-                if (hipGetLastError() != hipSuccess) st = FALM_ERR_HIP;
-                return spare;
-            }
-        }
         for (int it = 0; it < m; it++) {
             if (it > 0) {
                 TimedLaunch tm(FALM_TIME_SOR, s);
@@ -1968,8 +2021,8 @@ static T *pc_rest(falm_solver *S, const OP &a, T *x, const T *b, T *spare, hipSt
             hipLaunchKernelGGL((k_jacobi_op<T, OP>), FALM_GRID(S), s, S->tl, S->g, a, x, (const T *)S->w, b, done);
         }
     }
-    if (hipGetLastError() != hipSuccess) st = FALM_ERR_HIP;
-    return x;
+    FALM_CHECK_LAUNCH("pc_rest");
+    return FALM_OK;
 }
 
 // With the one-pass SOR preconditioner (pc_maxit <= 1) an iteration is the
@@ -2008,7 +2061,6 @@ static falm_status bicg_iteration(falm_solver *S, const OP &a, double *x, T *r, 
     const falm_solver_config &c = S->cfg;
     const Tiling &tl = S->tl;
     const Geom &g = S->g;
-    const int nb = S->kt.blocks;
     T *rr = (T *)S->rr, *p = (T *)S->p, *q = (T *)S->q, *sv = (T *)S->s, *pp = (T *)S->pp, *ss = (T *)S->ss,
       *t = (T *)S->t;
     const T wpc = (T)c.pc_relax;
@@ -2072,31 +2124,51 @@ static falm_status bicg_iteration(falm_solver *S, const OP &a, double *x, T *r, 
         FALM_CHECK_LAUNCH("k_fin_fold");
         return FALM_OK;
     }
-    falm_status pst;
-    hipLaunchKernelGGL((k_bicg_p<T, OP>), FALM_GRID(S), s, tl, g, a, (const T *)r, p, (const T *)q, pp,
-                       (const DevState *)S->st, c.pc_type, wpc);
+    // two SOR sweeps on a separable operator: the sweeps and the operator
+    // product are one kernel, which forms the first half-sweep itself
+    bool pc2 = false;
+    int nb = S->kt.blocks;
+    if constexpr (std::is_same<OP, OpSep<T>>::value) pc2 = c.pc_type == FALM_LS_SOR && c.pc_maxit == 2 && S->p2.blocks > 0;
+    const auto pc_mv = [&](auto mode, const T *b, const T *w, T *pc, T *o, double *partials) -> falm_status {
+        if constexpr (std::is_same<OP, OpSep<T>>::value) {
+            constexpr int M = decltype(mode)::value;
+            TimedLaunch tm(M == 1 ? FALM_TIME_PCMV : FALM_TIME_PCMV_S, s);
+            hipLaunchKernelGGL((k_bicg_pc2mv_km<T, M>), dim3((unsigned)S->p2.blocks), dim3(P2_NT), 0, s, S->p2, g, a, b,
+                               w, pc, o, (const DevState *)S->st, wpc, partials);
+            // v (and w) and the diagonal read, M(v) and A M(v) written
+            tm.done((double)tl.box.size() * ((M == 1 ? 5.0 : 4.0) * sizeof(T)));
+            FALM_CHECK_LAUNCH("k_bicg_pc2mv_km");
+        }
+        return FALM_OK;
+    };
+    if (pc2) nb = S->p2.blocks;
+    hipLaunchKernelGGL((k_bicg_p<T, OP>), FALM_GRID(S), s, tl, g, a, (const T *)r, p, (const T *)q,
+                       pc2 ? (T *)nullptr : pp, (const DevState *)S->st, c.pc_type, wpc);
     FALM_CHECK_LAUNCH("k_bicg_p");
-    // the preconditioned p lands in pp or, out of place, in w
-    T *const pcp = pc_rest<T, OP>(S, a, pp, p, (T *)S->w, s, pst);
-    FALM_TRY(pst);
-    TimedLaunch tm1(FALM_TIME_MV, s);
-    hipLaunchKernelGGL((k_bicg_mv_km<T, OP, 1>), FALM_KM(S), s, S->kt, g, a, (const T *)pcp, q, (const T *)rr,
-                       (const DevState *)S->st, S->partials);
-    tm1.done((double)tl.box.size() * (3.0 * sizeof(T) + diag_bytes<OP>(S)));
+    if (pc2) {
+        FALM_TRY(pc_mv(std::integral_constant<int, 1>{}, (const T *)p, (const T *)rr, pp, q, S->partials));
+    } else {
+        FALM_TRY((pc_rest<T, OP>(S, a, pp, p, s)));
+        TimedLaunch tm1(FALM_TIME_MV, s);
+        hipLaunchKernelGGL((k_bicg_mv_km<T, OP, 1>), FALM_KM(S), s, S->kt, g, a, (const T *)pp, q, (const T *)rr,
+                           (const DevState *)S->st, S->partials);
+        tm1.done((double)tl.box.size() * (3.0 * sizeof(T) + diag_bytes<OP>(S)));
+    }
     hipLaunchKernelGGL(k_fin_alpha, FALM_FIN, s, S->st, (const double *)S->partials, nb);
     FALM_CHECK_LAUNCH("k_bicg_mvdot");
-    hipLaunchKernelGGL((k_bicg_s<T, OP>), FALM_GRID(S), s, tl, g, a, (const T *)r, (const T *)q, sv, ss,
-                       (const DevState *)S->st, c.pc_type, wpc);
+    hipLaunchKernelGGL((k_bicg_s<T, OP>), FALM_GRID(S), s, tl, g, a, (const T *)r, (const T *)q, sv,
+                       pc2 ? (T *)nullptr : ss, (const DevState *)S->st, c.pc_type, wpc);
     FALM_CHECK_LAUNCH("k_bicg_s");
-    // the preconditioned s lands in ss or, out of place, in pp (free once
-    // p's sweeps have read it)
-    T *const pcs = pc_rest<T, OP>(S, a, ss, sv, pcp == pp ? ss : pp, s, pst);
-    FALM_TRY(pst);
-    TimedLaunch tm3(FALM_TIME_MV2, s);
-    hipLaunchKernelGGL((k_bicg_mv_km<T, OP, 2>), FALM_KM(S), s, S->kt, g, a, (const T *)pcs, t, (const T *)sv,
-                       (const DevState *)S->st, S->partials2);
-    tm3.done((double)tl.box.size() * (3.0 * sizeof(T) + diag_bytes<OP>(S)));
-    FALM_CHECK_LAUNCH("k_bicg_mvdot2");
+    if (pc2) {
+        FALM_TRY(pc_mv(std::integral_constant<int, 2>{}, (const T *)sv, (const T *)sv, ss, t, S->partials2));
+    } else {
+        FALM_TRY((pc_rest<T, OP>(S, a, ss, sv, s)));
+        TimedLaunch tm3(FALM_TIME_MV2, s);
+        hipLaunchKernelGGL((k_bicg_mv_km<T, OP, 2>), FALM_KM(S), s, S->kt, g, a, (const T *)ss, t, (const T *)sv,
+                           (const DevState *)S->st, S->partials2);
+        tm3.done((double)tl.box.size() * (3.0 * sizeof(T) + diag_bytes<OP>(S)));
+        FALM_CHECK_LAUNCH("k_bicg_mvdot2");
+    }
     // the pair update computes omega from mv2's partials itself (its own go
     // to the other buffer); the single-cell update reads it from the state
     const bool pairs = S->tp.tiles > 0 && ((uintptr_t)x & 15) == 0;
@@ -2106,11 +2178,11 @@ static falm_status bicg_iteration(falm_solver *S, const OP &a, double *x, T *r, 
     if (pairs) {
         nbu = S->tp.tiles < UPD_BLOCKS ? S->tp.tiles : UPD_BLOCKS;
         hipLaunchKernelGGL((k_bicg_update2<T>), dim3((unsigned)nbu), tiling_block(), 0, s, S->tp, tl.box.lo[0],
-                           g, x, (const T *)pcp, (const T *)pcs, (const T *)sv,
+                           g, x, (const T *)pp, (const T *)ss, (const T *)sv,
                            (const T *)t, r, (const T *)rr, (const DevState *)S->st, S->partials,
                            (const double *)S->partials2, nb, S->st);
     } else {
-        hipLaunchKernelGGL((k_bicg_update<T>), FALM_RED(S), s, tl, g, x, (const T *)pcp, (const T *)pcs,
+        hipLaunchKernelGGL((k_bicg_update<T>), FALM_RED(S), s, tl, g, x, (const T *)pp, (const T *)ss,
                            (const T *)sv, (const T *)t, r, (const T *)rr, (const DevState *)S->st, S->partials);
     }
     tm2.done((double)tl.box.size() * (2.0 * sizeof(double) + 6.0 * sizeof(T)));
@@ -2611,7 +2683,7 @@ falm_status falm_solver_create(const falm_domain *dom, const falm_solver_config 
         S->tp = make_tiling(pb);
         if (!even || S->tl.tiles == 0) S->tp.tiles = 0;
     }
-    S->s3 = make_s3_tiling(interior_box(S->g));
+    S->p2 = make_p2_tiling(interior_box(S->g));
     S->s2 = make_s2_tiling(interior_box(S->g));
     falm_status st = solver_alloc(S);
     if (st != FALM_OK) {
