@@ -63,7 +63,7 @@ def families():
         "sgs": (abi.TIME_SGS, "k_sgs_div (Smagorinsky + divergence + |div|^2)"),
         "divergence": (abi.TIME_DIVERGENCE, "k_div_norm (divergence + |div|^2)"),
         "solver_init": (abi.TIME_SOLVER_INIT, "k_bicg_init (b - A x in double + dots)"),
-        "sor": (abi.TIME_SOR, "k_sor_op_km / k_sor3_km (separate preconditioner sweeps, pc_maxit >= 2)"),
+        "sor": (abi.TIME_SOR, "k_sor_op_km (separate preconditioner sweeps, pc_maxit >= 2)"),
         "mv": (abi.TIME_MV, "k_bicg_mv_km<., ., 1> (q = A p^ + (rr, q); preconditioners other than one SOR pass)"),
         "mv2": (abi.TIME_MV2, "k_bicg_mv_km<., ., 2> (t = A s^ + (t, s), (t, t); the same)"),
         "pcmv": (abi.TIME_PCMV, "k_bicg_pcmv_km<., ., 0> (r = s - omega t, p = r + beta(p - omega q), "
