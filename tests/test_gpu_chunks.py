@@ -1,6 +1,6 @@
 """The k-marching kernels' chunk lengths: one plane a chunk on the smallest
 domains, a few on middle ones and a shorter last chunk, in the step driver
-(every stencil, the fused and the three-sweep preconditioner) against the
+(every stencil, the one- and the two-sweep preconditioner) against the
 oracle's steps.  The solve is cut at four iterations, where rounding has not
 been amplified (as in the solver tests): 1e-10, the step tests' bar."""
 import numpy as np
