@@ -374,7 +374,7 @@ __global__ __launch_bounds__(256) void k_adj_pseudo_u(Box xb, Geom g, double ALP
         }
     }
     // every store after every load (the compiler keeps their order)
-    if (nout == 0) {
+    if (nout == 0 && ffb.c[0]) {
 #pragma unroll
         for (int d = 0; d < 3; d++) ffb.c[d][c] = dt * own[d];
     }
@@ -385,6 +385,15 @@ __global__ __launch_bounds__(256) void k_adj_pseudo_u(Box xb, Geom g, double ALP
         if (ijk[d] < hi[d]) uunb.c[d][c] -= flx[d];
     }
     nutb[c] += nacc;
+}
+
+// ffb = dt uab on interior cells where the two are one buffer: after the
+// gather, whose threads read uab of their neighbours' cells
+__global__ void k_adj_scale_interior(Box ib, Geom g, double dt, F3 ffb) {
+    int i, j, k;
+    if (!box_cell(ib, gtid(), i, j, k)) return;
+    const int c = g.id(i, j, k);
+    for (int m = 0; m < 3; m++) ffb.c[m][c] *= dt;
 }
 
 // orc_sgs transposed, gathered over the interior grown by one cell (xb).
@@ -608,14 +617,18 @@ static F3 f3(void *p, size_t n) {
 static falm_status launch_adj_pseudo_u(const Geom &g, double ALPHA, double ReI, double dt, C3 u, C3 uu,
                                        const double *nut, C3 kx, C3 gg, const double *ja, C3 uab, F3 unb, F3 uunb,
                                        double *nutb, F3 ffb, hipStream_t s) {
-    const Box xb = grown_box(g, 2);
+    const Box xb = grown_box(g, 2), ib = interior_box(g);
+    const bool in_place = ffb.c[0] == uab.c[0];
+    const F3 ffk = in_place ? F3{} : ffb;  // the gather writes ffb unless it is uab itself
     const bool small = (size_t)g.nxy * (size_t)g.nz * sizeof(double) < (size_t(1) << 32);
     if (small)
         hipLaunchKernelGGL(k_adj_pseudo_u<unsigned>, box_grid(xb), dim3(EW_BLOCK), 0, s, xb, g, ALPHA, ReI, dt, u, uu,
-                           nut, kx, gg, ja, uab, unb, uunb, nutb, ffb);
+                           nut, kx, gg, ja, uab, unb, uunb, nutb, ffk);
     else
         hipLaunchKernelGGL(k_adj_pseudo_u<size_t>, box_grid(xb), dim3(EW_BLOCK), 0, s, xb, g, ALPHA, ReI, dt, u, uu,
-                           nut, kx, gg, ja, uab, unb, uunb, nutb, ffb);
+                           nut, kx, gg, ja, uab, unb, uunb, nutb, ffk);
+    if (in_place)
+        hipLaunchKernelGGL(k_adj_scale_interior, box_grid(ib), dim3(EW_BLOCK), 0, s, ib, g, dt, ffb);
     FALM_CHECK_LAUNCH("k_adj_pseudo_u");
     return FALM_OK;
 }

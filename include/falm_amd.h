@@ -469,7 +469,8 @@ falm_status falm_case_adjoint_attitude(falm_case *c, double *g_yaw, double *g_of
  *
  * falm_pseudo_u: adjoint w.r.t. u in both roles (un = u, as the step drivers
  * call it), uu, nut and ff; Upwind3, UTOPIA and KK only (else
- * FALM_ERR_UNSUPPORTED); ffbar is overwritten on interior cells (= dt uabar). */
+ * FALM_ERR_UNSUPPORTED); ffbar is overwritten on interior cells (= dt uabar)
+ * and may be uabar itself. */
 falm_status falm_pseudo_u_vjp(const falm_domain *dom, int adv_scheme, double ReI, double dt,
                               const void *u, const void *uu, const void *nut, const void *kx,
                               const void *g, const void *ja, const void *uabar, void *ubar,

@@ -207,6 +207,25 @@ def test_gathered_vjps_at_edges(gpu, n, sparse):
     assert rel_err(from_dev(ub), O.adj_sgs(dom, Cs, F["u"], F["kx"], F["ja"], wn) + had[0]) < TOL
 
 
+@pytest.mark.parametrize("n", [(5, 4, 3), (70, 21, 19)])
+def test_pseudo_u_vjp_in_place_ffbar(gpu, n):
+    """ffbar given as uabar's own buffer: the other adjoints as with a buffer
+    of its own, and the buffer's interior scaled by dt at the end (one
+    product a cell: exact)."""
+    dom = domain(n)
+    rng, F = _fields(dom, 78)
+    m, dt = interior_mask(dom, 3), 2e-3
+    w = rng.standard_normal(3 * dom.ncell)
+    d = {k: to_dev(v) for k, v in F.items()}
+    wd, out = to_dev(w), [to_dev(np.zeros(q * dom.ncell)) for q in (3, 3, 1)]
+    gpu.call("falm_pseudo_u_vjp", C.byref(dom), abi.ADV_UPWIND3, 1e-3, dt,
+             *_ptrs(gpu, d["u"], d["uu"], d["nut"], d["kx"], d["g"], d["ja"], wd, *out, wd), None)
+    ref = O.adj_pseudo_u(dom, 1 / 24, 1e-3, dt, F["u"], F["uu"], F["nut"], F["kx"], F["g"], F["ja"], w)
+    for a, b in zip(out, ref):
+        assert rel_err(from_dev(a), b) < TOL
+    assert np.array_equal(from_dev(wd), np.where(m, dt * w, w))
+
+
 def test_pseudo_u_vjp_rejects_other_schemes(gpu):
     dom = domain((6, 6, 6))
     z3, z1 = to_dev(np.zeros(3 * dom.ncell)), to_dev(np.zeros(dom.ncell))
