@@ -276,103 +276,123 @@ __global__ __launch_bounds__(256) void k_adj_pseudo_u(Box xb, Geom g, double ALP
         return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a) + (O)q * (O)sizeof(double));
     };
     const double rc = nout == 0 ? dt / ld(ja, c) : 0.0;
-    double acc[3] = {0.0, 0.0, 0.0}, nacc = 0.0;
-    double flx[3] = {0.0, 0.0, 0.0}, own[3] = {0.0, 0.0, 0.0};
+    double acc[3], nacc, flx[3], own[3] = {0.0, 0.0, 0.0};
     bool any = false;
     if (nout == 0) {
 #pragma unroll
-        for (int d = 0; d < 3; d++) acc[d] = own[d] = ld(uab.c[d], c);
+        for (int d = 0; d < 3; d++) own[d] = ld(uab.c[d], c);
     }
+    // MASK: a term whose adjoints are zero is left out, not multiplied, so
+    // that an operand which is not finite reaches only what depends on it
+    const auto gather = [&](auto mask) {
+        constexpr bool MASK = decltype(mask)::value;
+        const auto sel = [](bool use, double v) { return MASK && !use ? 0.0 : v; };
+        nacc = 0.0;
 #pragma unroll
-    for (int e = 0; e < 3; e++) {
-        const int s = st[e], p = ijk[e];
-        const bool out = p < g.gc || p >= hi[e];
-        if (nout > 0 && !out) continue;  // a ghost cell of another axis: no stencil along e
-        // every load is issued, at the nearest cell that has the value, and
-        // what lies outside is masked after: a load under a condition of its
-        // own waits for the one before it
-        bool in[5];
-        double w[5][3], W[5][3], A[5], JP[4], q[5][3];
-        bool live = false;
-        int at[5];
+        for (int d = 0; d < 3; d++) acc[d] = own[d], flx[d] = 0.0;
 #pragma unroll
-        for (int m = 0; m < 5; m++) {
-            const int v = p + m - 2;
-            in[m] = v >= g.gc && v < hi[e];
-            at[m] = c + ((v < g.gc ? g.gc : v >= hi[e] ? hi[e] - 1 : v) - p) * s;
-        }
+        for (int e = 0; e < 3; e++) {
+            const int s = st[e], p = ijk[e];
+            const bool out = p < g.gc || p >= hi[e];
+            if (nout > 0 && !out) continue;  // a ghost cell of another axis: no stencil along e
+            // every load is issued, at the nearest cell that has the value, and
+            // what lies outside is masked after: a load under a condition of its
+            // own waits for the one before it
+            bool in[5];
+            double w[5][3], W[5][3], A[5], JP[4], q[5][3];
+            bool live = false, on[5][3];
+            int at[5];
 #pragma unroll
-        for (int m = 0; m < 5; m++) {
-            if (m != 2) W[m][0] = ld(ja, at[m]);
+            for (int m = 0; m < 5; m++) {
+                const int v = p + m - 2;
+                in[m] = v >= g.gc && v < hi[e];
+                at[m] = c + ((v < g.gc ? g.gc : v >= hi[e] ? hi[e] - 1 : v) - p) * s;
+            }
 #pragma unroll
-            for (int d = 0; d < 3; d++) w[m][d] = ld(uab.c[d], at[m]);
-            A[m] = ld(kx.c[e], at[m]);
-        }
-        // u of the four or five cells that the faces below and above c and
-        // the fourth difference read, clamped to the array's own range
+            for (int m = 0; m < 5; m++) {
+                if (m != 2) W[m][0] = ld(ja, at[m]);
 #pragma unroll
-        for (int m = 0; m < 5; m++) {
-            const int v = p + m - 2, top = hi[e] + g.gc - 1;
-            const int f = c + ((v < 0 ? 0 : v > top ? top : v) - p) * s;
+                for (int d = 0; d < 3; d++) w[m][d] = ld(uab.c[d], at[m]);
+                A[m] = ld(kx.c[e], at[m]);
+            }
+            // u of the four or five cells that the faces below and above c and
+            // the fourth difference read, clamped to the array's own range
 #pragma unroll
-            for (int d = 0; d < 3; d++) q[m][d] = ld(u.c[d], f);
-            if (m < 4) JP[m] = ld(uu.c[e], f);
-            A[m] *= q[m][e];  // used where in[m]: f is the cell itself there
-        }
-        const int cp = c + (p + 1 <= hi[e] ? s : 0), cm = c - (p >= g.gc ? s : 0);
-        const double gc_ = ld(gg.c[e], c), gcp = ld(gg.c[e], cp), gcm = ld(gg.c[e], cm);
-        const double nc = ld(nut, c), ncp = ld(nut, cp), ncm = ld(nut, cm);
-        const double kc = ld(kx.c[e], c);
+            for (int m = 0; m < 5; m++) {
+                const int v = p + m - 2, top = hi[e] + g.gc - 1;
+                const int f = c + ((v < 0 ? 0 : v > top ? top : v) - p) * s;
 #pragma unroll
-        for (int m = 0; m < 5; m++) {
-            const double r = m == 2 ? rc : dt / W[m][0];
+                for (int d = 0; d < 3; d++) q[m][d] = ld(u.c[d], f);
+                if (m < 4) JP[m] = ld(uu.c[e], f);
+                A[m] *= q[m][e];  // used where in[m]: f is the cell itself there
+            }
+            const int cp = c + (p + 1 <= hi[e] ? s : 0), cm = c - (p >= g.gc ? s : 0);
+            const double gc_ = ld(gg.c[e], c), gcp = ld(gg.c[e], cp), gcm = ld(gg.c[e], cm);
+            const double nc = ld(nut, c), ncp = ld(nut, cp), ncm = ld(nut, cm);
+            const double kc = ld(kx.c[e], c);
+#pragma unroll
+            for (int m = 0; m < 5; m++) {
+                const double r = m == 2 ? rc : dt / W[m][0];
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    w[m][d] = in[m] ? w[m][d] : 0.0;
+                    on[m][d] = w[m][d] != 0.0;
+                    W[m][d] = sel(on[m][d], w[m][d] * r);
+                    live = live || on[m][d];
+                }
+            }
+            if (!live) continue;  // nothing to add, whatever the other operands are
+            any = true;
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const double co = m == 0 ? -1. : m == 1 ? 27. : m == 2 ? -27. : 1.;
+                const double J = (in[m] || in[m + 1]) ? JP[m] * (1. / 48.) : 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; d++) acc[d] -= co * (sel(on[m][d] || on[m + 1][d], J) * (W[m][d] + W[m + 1][d]));
+            }
+#pragma unroll
+            for (int m = 0; m < 5; m++) {
+                const double co = m == 2 ? 6. : (m == 1 || m == 3) ? -4. : 1.;
+                const double a = in[m] ? dt * ALPHA * fabs(A[m]) : 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; d++) acc[d] -= co * (sel(on[m][d], a) * w[m][d]);
+            }
+            const bool fp = in[2] || in[3], fm = in[1] || in[2];  // the faces above and below c
+            const double gp = fp ? 0.5 * (gc_ + gcp) : 0.0, gm = fm ? 0.5 * (gc_ + gcm) : 0.0;
+            const double Kp = fp ? gp * (ReI + 0.5 * (nc + ncp)) : 0.0;
+            const double Km = fm ? gm * (ReI + 0.5 * (nc + ncm)) : 0.0;
+            double fl = 0.0, sg4 = 0.0, np = 0.0, nm = 0.0;
+            bool onp = false, onm = false, on0 = false;
 #pragma unroll
             for (int d = 0; d < 3; d++) {
-                w[m][d] = in[m] ? w[m][d] : 0.0;
-                W[m][d] = w[m][d] * r;
-                live = live || w[m][d] != 0.0;
+                const bool op = on[2][d] || on[3][d], om = on[1][d] || on[2][d];
+                acc[d] += sel(op, Kp) * (W[3][d] - W[2][d]) - sel(om, Km) * (W[2][d] - W[1][d]);
+                fl += (W[2][d] + W[3][d]) * sel(op, 27 * (q[3][d] - q[2][d]) - (q[4][d] - q[1][d]));
+                np += sel(op, q[3][d] - q[2][d]) * (W[2][d] - W[3][d]);
+                nm += sel(om, q[1][d] - q[2][d]) * (W[2][d] - W[1][d]);
+                sg4 += w[2][d] * sel(on[2][d], q[4][d] - 4 * q[3][d] + 6 * q[2][d] - 4 * q[1][d] + q[0][d]);
+                onp = onp || op;
+                onm = onm || om;
+                on0 = on0 || on[2][d];
+            }
+            if (MASK ? onp : fp) {
+                nacc += 0.5 * gp * np;
+                flx[e] = fl * (1. / 48.);
+            }
+            if (MASK ? onm : fm) nacc += 0.5 * gm * nm;
+            if (MASK ? on0 : in[2]) {
+                const double U = A[2];
+                const double sg = (double)((U > 0) - (U < 0));
+                acc[e] -= dt * ALPHA * sg * kc * sg4;
             }
         }
-        if (!live) continue;  // nothing to add, whatever the other operands are
-        any = true;
+    };
+    gather(std::false_type{});
+    // without the mask such a term is 0 x Inf or 0 x NaN: it shows in a sum
+    double sum = nacc;
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const double co = m == 0 ? -1. : m == 1 ? 27. : m == 2 ? -27. : 1.;
-            const double J = (in[m] || in[m + 1]) ? JP[m] * (1. / 48.) : 0.0;
-#pragma unroll
-            for (int d = 0; d < 3; d++) acc[d] -= co * (J * (W[m][d] + W[m + 1][d]));
-        }
-#pragma unroll
-        for (int m = 0; m < 5; m++) {
-            const double co = m == 2 ? 6. : (m == 1 || m == 3) ? -4. : 1.;
-            const double a = in[m] ? dt * ALPHA * fabs(A[m]) : 0.0;
-#pragma unroll
-            for (int d = 0; d < 3; d++) acc[d] -= co * (a * w[m][d]);
-        }
-        const bool fp = in[2] || in[3], fm = in[1] || in[2];  // the faces above and below c
-        const double gp = fp ? 0.5 * (gc_ + gcp) : 0.0, gm = fm ? 0.5 * (gc_ + gcm) : 0.0;
-        const double Kp = fp ? gp * (ReI + 0.5 * (nc + ncp)) : 0.0;
-        const double Km = fm ? gm * (ReI + 0.5 * (nc + ncm)) : 0.0;
-        double fl = 0.0, sg4 = 0.0, np = 0.0, nm = 0.0;
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            acc[d] += Kp * (W[3][d] - W[2][d]) - Km * (W[2][d] - W[1][d]);
-            fl += (W[2][d] + W[3][d]) * (27 * (q[3][d] - q[2][d]) - (q[4][d] - q[1][d]));
-            np += (q[3][d] - q[2][d]) * (W[2][d] - W[3][d]);
-            nm += (q[1][d] - q[2][d]) * (W[2][d] - W[1][d]);
-            sg4 += w[2][d] * (q[4][d] - 4 * q[3][d] + 6 * q[2][d] - 4 * q[1][d] + q[0][d]);
-        }
-        if (fp) {
-            nacc += 0.5 * gp * np;
-            flx[e] = fl * (1. / 48.);
-        }
-        if (fm) nacc += 0.5 * gm * nm;
-        if (in[2]) {
-            const double U = A[2];
-            const double sg = (double)((U > 0) - (U < 0));
-            acc[e] -= dt * ALPHA * sg * kc * sg4;
-        }
-    }
+    for (int d = 0; d < 3; d++) sum += fabs(acc[d]) + fabs(flx[d]);
+    if (!isfinite(sum)) gather(std::true_type{});
     // every store after every load (the compiler keeps their order)
     if (nout == 0 && ffb.c[0]) {
 #pragma unroll

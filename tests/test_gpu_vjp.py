@@ -226,6 +226,43 @@ def test_pseudo_u_vjp_in_place_ffbar(gpu, n):
     assert np.array_equal(from_dev(wd), np.where(m, dt * w, w))
 
 
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_pseudo_u_vjp_leaves_out_zero_adjoints(gpu, bad):
+    """Where an adjoint component is zero its cell's operands do not count,
+    finite or not: with one component live at every sixth cell, the operands
+    that only the other cells (or components) read hold `bad` and every
+    output is the one without them."""
+    n = (26, 15, 9)
+    dom = domain(n)
+    rng, F = _fields(dom, 79)
+    nx, ny, nz = dom.shape
+    k, j, i = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    live = ((i + 2 * j + 3 * k) % 6 == 0) & interior_mask(dom).reshape(nz, ny, nx)
+    nc = dom.ncell
+    w = np.zeros(3 * nc)
+    w[:nc] = rng.standard_normal(nc) * live.ravel()
+
+    def reach(e, lo, hi):  # the cells m = lo .. hi along axis e of a live one
+        out = np.zeros_like(live)
+        for m in range(lo, hi + 1):
+            out |= np.roll(live, m, axis=2 - e)
+        return out
+
+    axes = range(3)
+    near = reach(0, -1, 1) | reach(1, -1, 1) | reach(2, -1, 1)
+    used = dict(u=[reach(0, -2, 2) | reach(1, -2, 2) | reach(2, -2, 2), live, live], uu=[reach(e, -1, 0) for e in axes],
+                nut=[near], kx=[live] * 3, g=[reach(e, -1, 1) for e in axes], ja=[live])
+    ref = O.adj_pseudo_u(dom, 1 / 24, 1e-3, 2e-3, F["u"], F["uu"], F["nut"], F["kx"], F["g"], F["ja"], w)
+    B = {q: np.where(np.concatenate([m.ravel() for m in ms]), F[q], bad) for q, ms in used.items()}
+    out = [to_dev(np.zeros(q * nc)) for q in (3, 3, 1, 3)]
+    d = {q: to_dev(v) for q, v in B.items()}
+    wd = to_dev(w)
+    gpu.call("falm_pseudo_u_vjp", C.byref(dom), abi.ADV_UPWIND3, 1e-3, 2e-3,
+             *_ptrs(gpu, d["u"], d["uu"], d["nut"], d["kx"], d["g"], d["ja"], wd, *out), None)
+    for a, b in zip(out, ref):
+        assert rel_err(from_dev(a), b) < TOL
+
+
 def test_pseudo_u_vjp_rejects_other_schemes(gpu):
     dom = domain((6, 6, 6))
     z3, z1 = to_dev(np.zeros(3 * dom.ncell)), to_dev(np.zeros(dom.ncell))
