@@ -6,10 +6,12 @@
 // Every stage is the transpose of the forward kernel it mirrors, computed in
 // double.  The stages over the whole field (projection, Poisson right-hand
 // side, face flux, pseudo-velocity, Smagorinsky) gather: each thread takes one
-// adjoint output cell and sums what the forward outputs that read it
-// contribute (deterministic, no atomics).  The boundary fills and the rotor
-// scatter over the forward's loop with hardware double atomics (their sums
-// are order-independent up to rounding).  The Poisson
+// adjoint output cell, sums in a fixed order what the forward outputs that
+// read it contribute, and adds that to the output once (pseudo-velocity and
+// Smagorinsky with an atomic add, so that calls on several streams may share
+// an output).  The boundary fills and the rotor scatter over the forward's
+// loop with hardware double atomics (their sums are order-independent up to
+// rounding).  The Poisson
 // solve is taken as exact; its adjoint is a BiCGStab solve with the
 // transposed operator.  Time is handled by checkpoints every `ckpt` steps and
 // recomputation of each segment's states during the reverse sweep.
@@ -251,11 +253,12 @@ __global__ void k_adj_fold_ghosts(Geom g, size_t n, F3 uab, F3 unb) {
 //                (g + g)/2 (1/Re + (nut + nut)/2)
 //   face flux    uub_e -= (W(0) + W(1))/2 L_d, L_d the face's difference
 //   viscosity    nutb += (g_c + g_f)/4 (u_d(f) - u_d(c)) (W(c) - W(f))
-// One thread per cell and no atomics, with 161 loads a cell that its
-// neighbours share in L1 and L2, where a scatter over forward cells makes 105
-// hardware atomic adds a cell: 2179 -> 315 us at 256 x 96 x 96.  L1 accesses
-// and FP64 instructions take about 90 us each; HBM would need 130 us for
-// the 34 values a cell.
+// One thread per cell, with 161 loads a cell that its neighbours share in L1
+// and L2 and one atomic add an output, where a scatter over forward cells makes
+// 105 of them a cell: 2179 -> 294 us at 256 x 96 x 96 (311 us with a load, an add
+// and a store in the atomic's place: the thread waits for that load).  L1
+// accesses and FP64 instructions take about 90 us each; HBM would need 130 us
+// for the 34 values a cell.
 // O: the type of a byte offset in a column (32 bits below 4 GiB: the loads then
 // share one offset register a cell instead of a 64-bit address each).
 template <class O>
@@ -401,10 +404,10 @@ __global__ __launch_bounds__(256) void k_adj_pseudo_u(Box xb, Geom g, double ALP
     if (!any) return;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        unb.c[d][c] += acc[d];
-        if (ijk[d] < hi[d]) uunb.c[d][c] -= flx[d];
+        unsafeAtomicAdd(&unb.c[d][c], acc[d]);
+        if (ijk[d] < hi[d]) unsafeAtomicAdd(&uunb.c[d][c], -flx[d]);
     }
-    nutb[c] += nacc;
+    unsafeAtomicAdd(&nutb[c], nacc);
 }
 
 // ffb = dt uab on interior cells where the two are one buffer: after the
@@ -425,9 +428,9 @@ __global__ void k_adj_scale_interior(Box ib, Geom g, double dt, F3 ffb) {
 // (double-buffered, one barrier a plane; the outermost threads only provide
 // theirs), while T_dz of the planes above and below stay in registers.  The
 // square root, the cube root and the division are so evaluated 1.4 times a
-// cell (6 times in a thread-per-cell gather), and no atomics are used: 263 ->
-// 116 us at 256 x 96 x 96 against the scatter's 18 atomic adds a cell.  It is
-// bound by the FP64 instructions of a plane (4.3 us with two workgroups a CU).
+// cell (6 times in a thread-per-cell gather), and an output takes one atomic
+// add against the scatter's 18 a cell: 264 -> 79 us at 256 x 96 x 96.  It is
+// bound by the FP64 instructions of a plane.
 constexpr int AS_X = 64, AS_Y = 8, AS_NT = AS_X * AS_Y;
 __global__ __launch_bounds__(AS_NT) void k_adj_sgs(Box xb, int tx, int ty, int kc, Geom g, double Cs, C3 u, C3 kx,
                                                    const double *__restrict__ ja, const double *__restrict__ nutb,
@@ -510,7 +513,7 @@ __global__ __launch_bounds__(AS_NT) void k_adj_sgs(Box xb, int tx, int ty, int k
             for (int d = 0; d < 3; d++) {
                 const double v = (lx[q][d][lj][li - 1] - lx[q][d][lj][li + 1]) +
                                  (ly[q][d][lj - 1][li] - ly[q][d][lj + 1][li]) + (tm[d] - T[d][2]);
-                if (v != 0.0) unb.c[d][c] += v;
+                if (v != 0.0) unsafeAtomicAdd(&unb.c[d][c], v);
             }
         }
 #pragma unroll

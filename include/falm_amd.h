@@ -457,10 +457,14 @@ falm_status falm_case_adjoint_attitude(falm_case *c, double *g_yaw, double *g_of
  * adjoint of a stage's output, each adds the adjoint of its inputs to the
  * *bar outputs (+=, so several contributions accumulate), except where
  * noted.  FP64 device arrays in the Matrix layout.  Whole-field stages add to
- * each output cell once, in a fixed order; the boundary fills and
- * falm_alm_vjp use atomics (order-independent to rounding, not bitwise
- * reproducible from run to run).  Calls that accumulate into the same output
- * must be ordered on one stream.
+ * each output cell once, a sum taken in a fixed order; the boundary fills and
+ * falm_alm_vjp add term by term (order-independent to rounding, not bitwise
+ * reproducible from run to run).  falm_pseudo_u_vjp, falm_sgs_vjp and
+ * falm_alm_vjp add atomically: calls on several streams may accumulate into
+ * one output.  The other stages' calls that share an output must be ordered
+ * (falm_project_p_vjp, falm_u_to_uu_vjp and falm_poisson_rhs_vjp add with a
+ * load and a store; falm_bc_velocity_vjp and falm_bc_pressure_vjp also
+ * overwrite).
  * The *bar outputs (and falm_alm_vjp's g_pitch, g_twist) must be device
  * memory from hipMalloc: the kernels accumulate into them with hardware FP64
  * atomic adds, which can drop updates on host-pinned, managed or

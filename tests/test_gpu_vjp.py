@@ -263,6 +263,34 @@ def test_pseudo_u_vjp_leaves_out_zero_adjoints(gpu, bad):
         assert rel_err(from_dev(a), b) < TOL
 
 
+def test_two_streams_add_to_one_output(gpu):
+    """Two streams that accumulate into the same outputs at once, pseudo-velocity
+    and Smagorinsky: nothing is lost.  24 terms of one size a sum: 1e-12."""
+    import torch
+    dom = domain((70, 40, 30))
+    rng, F = _fields(dom, 80)
+    d = {k: to_dev(v) for k, v in F.items()}
+    ws = [rng.standard_normal(3 * dom.ncell) for _ in range(2)]
+    wns = [rng.standard_normal(dom.ncell) for _ in range(2)]
+    wd, wnd = [to_dev(w) for w in ws], [to_dev(w) for w in wns]
+    out, ub = [to_dev(np.zeros(q * dom.ncell)) for q in (3, 3, 1)], to_dev(np.zeros(3 * dom.ncell))
+    ff = [to_dev(np.zeros(3 * dom.ncell)) for _ in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(12):
+        for q, s in enumerate(streams):
+            h = C.c_void_p(s.cuda_stream)
+            gpu.call("falm_pseudo_u_vjp", C.byref(dom), abi.ADV_UPWIND3, 1e-3, 2e-3,
+                     *_ptrs(gpu, d["u"], d["uu"], d["nut"], d["kx"], d["g"], d["ja"], wd[q], *out, ff[q]), h)
+            gpu.call("falm_sgs_vjp", C.byref(dom), 0.12, *_ptrs(gpu, d["u"], d["kx"], d["ja"], wnd[q], ub), h)
+    torch.cuda.synchronize()
+    ref = [O.adj_pseudo_u(dom, 1 / 24, 1e-3, 2e-3, F["u"], F["uu"], F["nut"], F["kx"], F["g"], F["ja"], w) for w in ws]
+    for q, a in enumerate(out):
+        assert rel_err(from_dev(a), 12 * (ref[0][q] + ref[1][q])) < TOL, q
+    refs = sum(O.adj_sgs(dom, 0.12, F["u"], F["kx"], F["ja"], w) for w in wns)
+    assert rel_err(from_dev(ub), 12 * refs) < TOL
+
+
 def test_pseudo_u_vjp_rejects_other_schemes(gpu):
     dom = domain((6, 6, 6))
     z3, z1 = to_dev(np.zeros(3 * dom.ncell)), to_dev(np.zeros(dom.ncell))
