@@ -1923,6 +1923,7 @@ static falm_status solver_alloc(falm_solver *S) {
     size_t nb = (size_t)(S->tl.tiles > 0 ? red_blocks(S->tl) : 1);
     if ((size_t)S->kt.blocks > nb) nb = (size_t)S->kt.blocks;
     if ((size_t)S->ktp.blocks > nb) nb = (size_t)S->ktp.blocks;
+    if ((size_t)S->p2.blocks > nb) nb = (size_t)S->p2.blocks;
     if ((size_t)S->s2.blocks * s2_k(S->s2) > 2 * nb) nb = (size_t)S->s2.blocks * s2_k(S->s2) / 2 + 1;  // k_sor2d's norms
     FALM_HIP(hipMalloc(&S->partials, 2 * nb * sizeof(double)));
     FALM_HIP(hipMalloc(&S->trash, (size_t)(S->ktp.blocks > 0 ? S->ktp.blocks : 1) * K7_NT * 2 * sizeof(double)));
