@@ -835,9 +835,10 @@ inline int p2_tiles(int n, int region) {
     const int rest = n - 2 * (region - P2_R), o = region - 2 * P2_R;
     return 2 + (rest > 0 ? (rest + o - 1) / o : 0);
 }
-// One double workgroup runs on a CU (162 VGPRs, 115 KB of LDS), so the time is the rounds of 256
-// workgroups times a chunk's steps; a chunk of n planes takes n + 11, of which
-// the first six and the last two do one half-sweep pair of the two.
+// One double workgroup runs on a CU (164 VGPRs, 115 KB of LDS), so the time is
+// the rounds of 256 workgroups times a chunk's steps; a chunk of n planes takes
+// n + 11 (n + 7 at the domain's lower end), of which the first six and the last
+// two do one half-sweep pair of the two.
 inline P2Tiling make_p2_tiling(const Box &b) {
     P2Tiling t;
     t.box = b;
@@ -918,8 +919,13 @@ __global__ __launch_bounds__(P2_NT) __attribute__((amdgpu_waves_per_eu(P2_NW / 4
         pub[s][f][0][c][l] = T(0);
         pub[s][f][P2_NW + 1][c][l] = T(0);
     }
-    // s0: the first step; blk0: column 0's cell is black at plane s0
-    const int s0 = k0 - 6;
+    // s0: the first step.  Outside the domain every half-sweep is zero, so a
+    // chunk at its start makes no step below it, and a pair of half-sweeps
+    // whose planes both lie outside is passed over: a domain of one plane is
+    // left with two steps of each pair of 12 (a solve of 6 iterations in double
+    // at 128 x 128 x 1 310 -> 249 us, at 512 x 512 x 1 487 -> 362, x 4 708 -> 599).
+    // blk0: column 0's cell is black at plane s0
+    const int s0 = max(k0 - 6, lo2 - 2);
     const bool blk0 = ((i + j0 + s0 + g.osum) & 1) == FALM_COLOR_BLACK;
     T X1[C][4], X2[C][4], V[C][4], D[C][4], nv[C], nd[C], nw[C], na[C];
 #pragma unroll
@@ -972,8 +978,7 @@ __global__ __launch_bounds__(P2_NT) __attribute__((amdgpu_waves_per_eu(P2_NW / 4
                 na[r] = ld_at(a.ac, ob);
             }
         }
-        if (s <= k1 + 2) {
-            const bool kb = kin(s + 2), kr = kin(s);
+        if (const bool kb = kin(s + 2), kr = kin(s); s <= k1 + 2 && (kb || kr)) {
 #pragma unroll
             for (int r = 0; r < C; r++) {
                 const bool b = (r & 1) ? !b0 : b0;
@@ -990,23 +995,27 @@ __global__ __launch_bounds__(P2_NT) __attribute__((amdgpu_waves_per_eu(P2_NW / 4
             const bool kb = kin(s - 2), kr = kin(s - 4);
             T y[C], x2[C];
 #pragma unroll
-            for (int r = 0; r < C; r++) {
-                const bool b = (r & 1) ? !b0 : b0;
-                y[r] = b ? X2[r][m2] : X1[r][m2];
-            }
+            for (int r = 0; r < C; r++) x2[r] = T(0);
+            if (kb || kr) {
 #pragma unroll
-            for (int r = 0; r < C; r++) {
-                const bool b = (r & 1) ? !b0 : b0;
-                // beyond the thread's rows the neighbour has the other colour
-                const T xn = r + 1 < C ? y[r + 1 < C ? r + 1 : r] : (b ? u1 : u2);
-                const T xs = r > 0 ? y[r > 0 ? r - 1 : 0] : (b ? l1 : l2);
-                const T xc = X1[r][q];
-                const T sum = D[r][q] * xc + ae * p2_shift<0x130>(y[r]) + aw * p2_shift<0x138>(y[r]) + an[r] * xn +
-                              as[r] * xs + (b ? at[2] : at[4]) * (b ? X1[r][m1] : X2[r][m1]) +
-                              (b ? ab[2] : ab[4]) * (b ? X1[r][m3] : X2[r][m3]);
-                T x = xc + omega_pc * ((V[r][q] - sum) / D[r][q]);
-                p2_keep(x);
-                x2[r] = in[r] && (b ? kb : kr) ? x : T(0);
+                for (int r = 0; r < C; r++) {
+                    const bool b = (r & 1) ? !b0 : b0;
+                    y[r] = b ? X2[r][m2] : X1[r][m2];
+                }
+#pragma unroll
+                for (int r = 0; r < C; r++) {
+                    const bool b = (r & 1) ? !b0 : b0;
+                    // beyond the thread's rows the neighbour has the other colour
+                    const T xn = r + 1 < C ? y[r + 1 < C ? r + 1 : r] : (b ? u1 : u2);
+                    const T xs = r > 0 ? y[r > 0 ? r - 1 : 0] : (b ? l1 : l2);
+                    const T xc = X1[r][q];
+                    const T sum = D[r][q] * xc + ae * p2_shift<0x130>(y[r]) + aw * p2_shift<0x138>(y[r]) + an[r] * xn +
+                                  as[r] * xs + (b ? at[2] : at[4]) * (b ? X1[r][m1] : X2[r][m1]) +
+                                  (b ? ab[2] : ab[4]) * (b ? X1[r][m3] : X2[r][m3]);
+                    T x = xc + omega_pc * ((V[r][q] - sum) / D[r][q]);
+                    p2_keep(x);
+                    x2[r] = in[r] && (b ? kb : kr) ? x : T(0);
+                }
             }
             if (k >= k0) {
                 T c[C];

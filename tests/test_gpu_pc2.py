@@ -24,7 +24,8 @@ def separable(dom, rng):
     return np.concatenate([c.reshape(-1) for c in (diag, *off)])
 
 
-@pytest.mark.parametrize("n", [(64, 24, 1), (65, 25, 2), (120, 40, 9), (121, 41, 5), (7, 81, 31), (180, 3, 64), (127, 4, 64)])
+@pytest.mark.parametrize("n", [(64, 24, 1), (65, 25, 2), (120, 40, 9), (121, 41, 5), (7, 81, 31), (180, 3, 64), (127, 4, 64),
+                               (600, 470, 1), (130, 70, 3), (66, 100, 4)])
 @pytest.mark.parametrize("offset", [(0, 0, 0), (1, 2, 4)])
 @pytest.mark.parametrize("precision", [abi.SOLVE_F64, abi.SOLVE_MIXED])
 def test_two_sweeps_at_edges(gpu, n, offset, precision):
