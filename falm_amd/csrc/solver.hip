@@ -851,7 +851,7 @@ inline P2Tiling make_p2_tiling(const Box &b) {
     long best = LONG_MAX;
     for (int kc = 1; kc <= b.n[2]; kc++) {
         const long tk = (b.n[2] + kc - 1) / kc;
-        if (cols * tk > RED_BLOCKS) continue;
+        if (tk > 1 && cols * tk > RED_BLOCKS) continue;  // beyond that many columns: whole ones
         const long cost = ((cols * tk + 255) / 256) * (kc + 7);
         if (cost >= best) continue;
         best = cost;

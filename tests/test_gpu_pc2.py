@@ -51,3 +51,22 @@ def test_two_sweeps_at_edges(gpu, n, offset, precision):
         assert rel_err(from_dev(dx), x_ref) < bar, declared
         if precision == abi.SOLVE_F64:
             assert rel_err(from_dev(dr), r_ref) < 1e-9
+
+
+@pytest.mark.parametrize("precision", [abi.SOLVE_F64, abi.SOLVE_MIXED])
+def test_two_sweeps_beyond_4096_columns(gpu, precision):
+    """41 x 106 = 4346 tiles of whole columns, more than a reduction's usual
+    number of partial sums: the oracle's first iterations as above."""
+    dom = domain((2300, 1700, 1))
+    rng = np.random.default_rng(9)
+    a, m = separable(dom, rng), interior_mask(dom)
+    b = rng.standard_normal(dom.ncell) * m
+    cfg = abi.solver_config(maxit=2, tol=1e-30, pc_type=abi.LS_SOR, pc_maxit=2, pc_relax=1.3, precision=precision)
+    x_ref, r_ref = np.zeros(dom.ncell), np.zeros(dom.ncell)
+    info_ref = O.Solver(dom, cfg).solve(a, x_ref, b, r_ref)
+    S = gpu.Solver(dom, cfg)
+    da, db, dx = to_dev(a), to_dev(b), to_dev(np.zeros(dom.ncell))
+    S.set_matrix(da)
+    info = S.solve(da, dx, db, None)
+    assert info.it == info_ref.it == 2
+    assert rel_err(from_dev(dx), x_ref) < (1e-11 if precision == abi.SOLVE_F64 else 2e-5)
