@@ -457,9 +457,9 @@ falm_status falm_case_adjoint_attitude(falm_case *c, double *g_yaw, double *g_of
  * adjoint of a stage's output, each adds the adjoint of its inputs to the
  * *bar outputs (+=, so several contributions accumulate), except where
  * noted.  FP64 device arrays in the Matrix layout.  Whole-field stages add to
- * each output cell once, a sum taken in a fixed order; the boundary fills and
- * falm_alm_vjp add term by term (order-independent to rounding, not bitwise
- * reproducible from run to run).  falm_pseudo_u_vjp, falm_sgs_vjp and
+ * each output cell once, a sum taken in a fixed order; the boundary fills,
+ * falm_alm_vjp and falm_sgs_vjp on domains below 90 000 cells add term by term
+ * (order-independent to rounding, not bitwise reproducible from run to run).  falm_pseudo_u_vjp, falm_sgs_vjp and
  * falm_alm_vjp add atomically: calls on several streams may accumulate into
  * one output.  The other stages' calls that share an output must be ordered
  * (falm_project_p_vjp, falm_u_to_uu_vjp and falm_poisson_rhs_vjp add with a

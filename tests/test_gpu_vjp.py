@@ -175,9 +175,11 @@ def test_pseudo_u_vjp(gpu, scheme):
     assert abs(fd - ad) <= 1e-6 * abs(fd)
 
 
-# one cell; thin boxes; the Smagorinsky tile's last output column and row
-# (60 + 2 = 62, 4 + 2 = 6) and one beyond; several chunks of planes
-@pytest.mark.parametrize("n", [(1, 1, 1), (2, 3, 1), (60, 4, 5), (61, 5, 3), (130, 13, 40)])
+# one cell; thin boxes; several chunks of planes.  From 90 000 cells on the
+# Smagorinsky transpose walks tiles of planes: its last output column and row
+# (60 + 2 = 62, 40 + 2 = 7 x 6) and one beyond, two full tiles, thin boxes
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 3, 1), (60, 4, 5), (61, 5, 3), (130, 13, 40), (60, 40, 38), (61, 41, 37),
+                               (122, 10, 75), (2, 215, 210), (300, 301, 1)])
 @pytest.mark.parametrize("sparse", [False, True])
 def test_gathered_vjps_at_edges(gpu, n, sparse):
     """The gathered pseudo-velocity and Smagorinsky transposes where their
@@ -263,11 +265,13 @@ def test_pseudo_u_vjp_leaves_out_zero_adjoints(gpu, bad):
         assert rel_err(from_dev(a), b) < TOL
 
 
-def test_two_streams_add_to_one_output(gpu):
+@pytest.mark.parametrize("n", [(70, 40, 30), (70, 45, 40)])
+def test_two_streams_add_to_one_output(gpu, n):
     """Two streams that accumulate into the same outputs at once, pseudo-velocity
-    and Smagorinsky: nothing is lost.  24 terms of one size a sum: 1e-12."""
+    and Smagorinsky (n: its scatter, its walk): nothing is lost.  24 terms of
+    one size a sum: 1e-12."""
     import torch
-    dom = domain((70, 40, 30))
+    dom = domain(n)
     rng, F = _fields(dom, 80)
     d = {k: to_dev(v) for k, v in F.items()}
     ws = [rng.standard_normal(3 * dom.ncell) for _ in range(2)]
