@@ -124,6 +124,10 @@ __global__ void k_adj_ubc(Geom g, FaceRange fr, const double *xyz0, double dt, C
 // with weight -+ dt/2 kx_d, its face part on the face region (fb) reads p at
 // f + e_d and f with weight -+ dt/2 (g_d(f) + g_d(f + e_d)); p's adjoint at
 // c sums those terms of the cells whose stencils reach c
+// SHARED: outputs that share memory are added to one after the other
+// (otherwise their old values are loaded with the operands: 107 us at 256 x 96
+// x 96, 116 with atomic adds).
+template <bool SHARED>
 __global__ void k_adj_project(Box xb, Box fb, Box ib, Geom g, double dt, C3 kx, C3 gg, C3 usb, C3 uunb, F3 uab,
                               F3 uusb, double *pb) {
     int i, j, k;
@@ -148,14 +152,21 @@ __global__ void k_adj_project(Box xb, Box fb, Box ib, Geom g, double dt, C3 kx, 
         ggv[d][0] = gg.c[d][cm];
         ggv[d][1] = gg.c[d][c];
         ggv[d][2] = gg.c[d][cp];
-        ua[d] = uab.c[d][c];
-        uua[d] = uusb.c[d][c];
+        if (!SHARED) {
+            ua[d] = uab.c[d][c];
+            uua[d] = uusb.c[d][c];
+        }
     }
-    const double p0 = pb[c];
+    const double p0 = SHARED ? 0.0 : pb[c];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        if (cin) uab.c[d][c] = ua[d] + us[d][1];
-        if (cf) uusb.c[d][c] = uua[d] + uf[d][1];
+        if (SHARED) {
+            if (cin) unsafeAtomicAdd(&uab.c[d][c], us[d][1]);
+            if (cf) unsafeAtomicAdd(&uusb.c[d][c], uf[d][1]);
+        } else {
+            if (cin) uab.c[d][c] = ua[d] + us[d][1];
+            if (cf) uusb.c[d][c] = uua[d] + uf[d][1];
+        }
         const bool mi = in_box(ib, i - (d == 0), j - (d == 1), k - (d == 2));
         const bool pi = in_box(ib, i + (d == 0), j + (d == 1), k + (d == 2));
         const bool mf = in_box(fb, i - (d == 0), j - (d == 1), k - (d == 2));
@@ -164,7 +175,8 @@ __global__ void k_adj_project(Box xb, Box fb, Box ib, Geom g, double dt, C3 kx, 
         acc -= mf ? dt * 0.5 * (ggv[d][0] + ggv[d][1]) * uf[d][0] : 0.0;
         acc += cf ? dt * 0.5 * (ggv[d][1] + ggv[d][2]) * uf[d][1] : 0.0;
     }
-    pb[c] = p0 + acc;
+    if (SHARED) unsafeAtomicAdd(&pb[c], acc);
+    else pb[c] = p0 + acc;
 }
 
 // orc_bc_pressure transposed: Neumann ghost = interior neighbour, ZERO = 0
@@ -820,9 +832,12 @@ falm_status falm_project_p_vjp(const falm_domain *dom, double dt, const void *kx
     const Geom gm = make_geom(dom);
     const size_t n = ncell_of(dom);
     const Box fb = face_box(gm), ib = interior_box(gm), xb = ext_box(gm);
-    hipLaunchKernelGGL(k_adj_project, box_grid(xb), dim3(EW_BLOCK), 0, (hipStream_t)stream, xb, fb, ib, gm, dt,
-                       c3(kx, n), c3(g, n), c3(ubar, n), c3(uubar, n), f3(uabar, n), f3(uuabar, n),
-                       (double *)pbar);
+    const size_t vb = 3 * n * sizeof(double), sb = n * sizeof(double);
+    const bool shared =
+        overlaps(uabar, vb, uuabar, vb) || overlaps(uabar, vb, pbar, sb) || overlaps(uuabar, vb, pbar, sb);
+    hipLaunchKernelGGL(shared ? k_adj_project<true> : k_adj_project<false>, box_grid(xb), dim3(EW_BLOCK), 0,
+                       (hipStream_t)stream, xb, fb, ib, gm, dt, c3(kx, n), c3(g, n), c3(ubar, n), c3(uubar, n),
+                       f3(uabar, n), f3(uuabar, n), (double *)pbar);
     FALM_CHECK_LAUNCH("k_adj_project");
     return FALM_OK;
 }
@@ -1012,7 +1027,7 @@ falm_status falm_case_adjoint(falm_case *C, int nsteps, int ckpt, double adj_rto
             hipLaunchKernelGGL(k_adj_copy_interior, box_grid(ib), dim3(EW_BLOCK), 0, s, ib, g, c3(ub, n), f3(usb, n));
             hipLaunchKernelGGL(k_adj_ubc, ew_grid((size_t)nvf), dim3(EW_BLOCK), 0, s, g, vfr, (const double *)C->xyz,
                                c.dt, c3(ub, n), f3(usb, n), f3(unb, n));
-            hipLaunchKernelGGL(k_adj_project, box_grid(xbx), dim3(EW_BLOCK), 0, s, xbx, fbx, ib, g, c.dt, kx, gg,
+            hipLaunchKernelGGL(k_adj_project<false>, box_grid(xbx), dim3(EW_BLOCK), 0, s, xbx, fbx, ib, g, c.dt, kx, gg,
                                c3(usb, n), c3(uub, n), f3(uab, n), f3(uusb, n), pb);
             hipLaunchKernelGGL(k_adj_pbc, ew_grid((size_t)npf), dim3(EW_BLOCK), 0, s, g, pfr, pb);
             FALM_CHECK_LAUNCH("k_adj_pbc");

@@ -1491,11 +1491,6 @@ static MetSep<T> met_sep(const SepMesh &sm) {
     return m;
 }
 
-static bool overlaps(const void *a, size_t abytes, const void *b, size_t bbytes) {
-    const char *x = (const char *)a, *y = (const char *)b;
-    return x < y + bbytes && y < x + abytes;
-}
-
 template <class T, class M>
 static falm_status pseudo_u_t(const falm_domain *dom, int scheme, double ReI, double dt, const void *un,
                               const void *u, const void *uu, void *ua, const void *nut, const M &met,

@@ -353,6 +353,11 @@ template <> struct PrecOf<float> { static constexpr int value = FALM_F32; };
 
 inline size_t prec_bytes(int prec) { return prec == FALM_F32 ? 4 : 8; }
 
+inline bool overlaps(const void *a, size_t abytes, const void *b, size_t bbytes) {
+    const char *x = (const char *)a, *y = (const char *)b;
+    return x < y + bbytes && y < x + abytes;
+}
+
 // column pointer helper
 template <class T> inline T *col(void *p, size_t ncell, int c) { return (T *)p + (size_t)c * ncell; }
 template <class T> inline const T *col(const void *p, size_t ncell, int c) {

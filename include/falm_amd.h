@@ -485,7 +485,8 @@ falm_status falm_u_to_uu_vjp(const falm_domain *dom, const void *kx, const void 
 /* falm_poisson_rhs: rhsbar (interior) -> uubar */
 falm_status falm_poisson_rhs_vjp(const falm_domain *dom, const void *ja, double dt, double maxdiag,
                                  const void *rhsbar, void *uubar, void *stream);
-/* falm_project_p: (ubar, uubar) of the outputs -> uabar, uuabar, pbar */
+/* falm_project_p: (ubar, uubar) of the outputs -> uabar, uuabar, pbar (which
+ * may share memory) */
 falm_status falm_project_p_vjp(const falm_domain *dom, double dt, const void *kx, const void *g,
                                const void *ubar, const void *uubar, void *uabar, void *uuabar,
                                void *pbar, void *stream);

@@ -90,6 +90,19 @@ def test_poisson_rhs_vjp(gpu):
     assert abs(lhs - rh) <= 1e-12 * abs(lhs)
 
 
+def test_project_p_vjp_into_one_output(gpu):
+    """uabar and uuabar given as one buffer: it gets both adjoints' sum."""
+    dom = domain(N)
+    rng, F = _fields(dom, 81)
+    ub = rng.standard_normal(3 * dom.ncell) * interior_mask(dom, 3)
+    uub = rng.standard_normal(3 * dom.ncell) * _face_mask(dom, 3)
+    ra, rua, rp = O.adj_project(dom, 3e-3, F["kx"], F["g"], ub, uub)
+    kx, g, ubd, uubd = (to_dev(v) for v in (F["kx"], F["g"], ub, uub))
+    a, p = to_dev(np.zeros(3 * dom.ncell)), to_dev(np.zeros(dom.ncell))
+    gpu.call("falm_project_p_vjp", C.byref(dom), 3e-3, *_ptrs(gpu, kx, g, ubd, uubd, a, a, p), None)
+    assert rel_err(from_dev(a), ra + rua) < TOL and rel_err(from_dev(p), rp) < TOL
+
+
 def test_project_p_vjp(gpu):
     dom = domain(N)
     rng, F = _fields(dom, 3)
