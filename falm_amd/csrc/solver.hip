@@ -1551,10 +1551,13 @@ __global__ __launch_bounds__(FIN_NT) void k_fin_resnorm(DevState *st, const doub
 // home.
 //
 // Measured at 128 x 128: a launch takes 7 us (3 of them that of an empty one;
-// the rest loads, the norms' sums) and 0.6 to 1 us an iteration: 10 us at
-// K = 4, 11.2 at 6, 12.2 at 7.  More iterations need a wider ring, so the
-// smallest domains take the most: the line lies where each workgroup sums all
-// partials and every workgroup finds a CU of its own.
+// the rest loads, the norms' sums) and 0.7 to 1.1 us an iteration: 10 us at
+// K = 4, 11.2 at 6, 12.2 at 7, and 0.8 at 7 for the division (those figures are
+// with a product by the stored reciprocal and one fused correction, which is not
+// always the rounded quotient and not one at all for infinite or tiny values).
+// More iterations need a wider ring, so the smallest domains take the most: the
+// line lies where each workgroup sums all partials and every workgroup finds a
+// CU of its own.
 template <int K_, int TX_, int TY_, int MAXWG_>
 struct S2Cfg {
     static constexpr int K = K_, TX = TX_, TY = TY_, MAXWG = MAXWG_, NT = 1024;
@@ -1591,20 +1594,13 @@ inline int s2_k(const S2Tiling &t) { return t.cfg == 0 ? S2A::K : t.cfg == 1 ? S
 
 // One cell of the region: its coefficients, x, and b without the two z
 // neighbours' products, which do not change.  The residual is summed as a
-// tree and the division is a product with the stored reciprocal corrected by
-// one fused step (correctly rounded but for ties of two ulps): a half-sweep is
-// one chain of dependent double operations, 7 this way, 28 as a running sum
-// and a division.
+// tree: a half-sweep is one chain of dependent double operations.
 struct S2Cell {
-    double ac, aw, ae, as, an, b, x, ra;
+    double ac, aw, ae, as, an, b, x;
     int cc;
     bool inner, upd, out;  // an interior cell; updated here; in the tile (stored and counted)
     __device__ inline double res(double xe, double xw, double xn, double xs) const {
         return fma(-ac, x, b) - (fma(aw, xw, ae * xe) + fma(as, xs, an * xn));
-    }
-    __device__ inline double over_ac(double v) const {
-        const double q = v * ra;
-        return fma(fma(-ac, q, v), ra, q);
     }
 };
 
@@ -1657,7 +1653,6 @@ __global__ __launch_bounds__(C::NT) void k_sor2d(S2Tiling tl, Geom g, OP a, doub
         c.an = q.an;
         c.x = q.x;
         c.b = fma(-q.ab, q.xb, fma(-q.at, q.xt, q.b));
-        c.ra = 1.0 / q.ac;
     };
     S2Cell cb, cr;
     Raw qb, qr;
@@ -1722,7 +1717,7 @@ __global__ __launch_bounds__(C::NT) void k_sor2d(S2Tiling tl, Geom g, OP a, doub
             const double rv = cb.res(lx[1][wb + 1], lx[1][wb], lx[1][nn], lx[1][sn]);
             if (m > 0 && cb.out) acc[m - 1] += rv * rv;
             if (m < mrun) {
-                cb.x = cb.x + omega * cb.over_ac(rv);
+                cb.x = cb.x + omega * (rv / cb.ac);
                 lx[0][tid] = cb.x;
             }
         }
@@ -1730,7 +1725,7 @@ __global__ __launch_bounds__(C::NT) void k_sor2d(S2Tiling tl, Geom g, OP a, doub
         __syncthreads();
         if (cr.upd) {
             const double xe = lx[0][wr + 1], xv = lx[0][wr], xn = lx[0][nn], xs = lx[0][sn];
-            cr.x = cr.x + omega * cr.over_ac(cr.res(xe, xv, xn, xs));
+            cr.x = cr.x + omega * (cr.res(xe, xv, xn, xs) / cr.ac);
             lx[1][tid] = cr.x;
             if (cr.out) {
                 const double rv = cr.res(xe, xv, xn, xs);

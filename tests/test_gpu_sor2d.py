@@ -78,3 +78,25 @@ def test_sor_one_layer_stops_and_goes_on(gpu):
             info = one.solve(da, dx, db, dr)
             assert info.it == i_ref.it and info.status == i_ref.status == abi.FALM_OK, tol
             assert rel_err(from_dev(dx), x_ref) < 1e-10
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf])
+@pytest.mark.parametrize("at", [(9, 8), (10, 8)])  # a black and a red cell
+def test_sor_one_layer_infinite_value(gpu, bad, at):
+    """An infinite right-hand side value makes infinite, not undefined, x where
+    the sweep's expression does: the oracle's iterate of the one iteration
+    after which the residual is undefined, cell by cell."""
+    dom, a, x0, b, m = _system((20, 16, 1), 2, (0, 0, 0), 7)
+    nx, ny, _ = dom.shape
+    b[at[0] + nx * (at[1] + ny * dom.gc)] = bad
+    cfg = abi.solver_config(type=abi.LS_SOR, maxit=5, tol=1e-30, relax=1.3, pc_type=abi.LS_EMPTY)
+    x_ref, r_ref = x0.copy(), np.zeros(dom.ncell)
+    with np.errstate(all="ignore"):
+        i_ref = O.Solver(dom, cfg).solve(a, x_ref, b, r_ref)
+    dx = to_dev(x0)
+    info = gpu.Solver(dom, cfg).solve(to_dev(a), dx, to_dev(b), to_dev(np.zeros(dom.ncell)))
+    got, fin = from_dev(dx), np.isfinite(x_ref)
+    assert info.it == i_ref.it == 1 and np.isnan(info.err)
+    assert np.isinf(x_ref).any() and not np.isnan(x_ref).any()
+    assert np.array_equal(got[~fin], x_ref[~fin])
+    assert np.max(np.abs(got[fin] - x_ref[fin])) < 1e-12 * np.max(np.abs(x_ref[fin]))
