@@ -2411,7 +2411,10 @@ template <class OP>
 static falm_status solve_stationary(falm_solver *S, const OP &a, double *x, const double *b, double *r,
                                     hipStream_t s, falm_solve_info *info, int mode) {
     const falm_solver_config &c = S->cfg;
-    if (c.type == FALM_LS_SOR && S->s2.blocks > 0) return solve_sor2d(S, a, x, b, r, s, info, mode);
+    // one layer: several iterations a launch, unless there is only one (it then
+    // takes a second launch that finds the solve over: 41 us at 128 x 128
+    // against 33; two iterations 42 against 65)
+    if (c.type == FALM_LS_SOR && S->s2.blocks > 0 && c.maxit > 1) return solve_sor2d(S, a, x, b, r, s, info, mode);
     const int period = check_period(S);
     const int *done = &S->st->done;
     const int nb = red_blocks(S->tl);
