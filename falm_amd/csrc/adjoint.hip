@@ -715,9 +715,8 @@ static falm_status launch_adj_sgs(const Geom &g, double Cs, C3 u, C3 kx, const d
         return FALM_OK;
     }
     const int tx = (xb.n[0] + AS_X - 3) / (AS_X - 2), ty = (xb.n[1] + AS_Y - 3) / (AS_Y - 2);
-    // one round of workgroups, two to a CU (128 VGPRs)
-    const int want = 512 / (tx * ty) > 0 ? 512 / (tx * ty) : 1;
-    const int kc = (xb.n[2] + want - 1) / want, tk = (xb.n[2] + kc - 1) / kc;
+    // two workgroups to a CU (128 VGPRs), two planes more than a chunk holds
+    const int kc = k7_chunk_rounds(tx * ty, xb.n[2], 2 * cu_count(), 2), tk = (xb.n[2] + kc - 1) / kc;
     hipLaunchKernelGGL(k_adj_sgs, dim3((unsigned)(tx * ty * tk)), dim3(AS_NT), 0, s, xb, tx, ty, kc, g, Cs, u, kx, ja,
                        nutb, unb);
     FALM_CHECK_LAUNCH("k_adj_sgs");

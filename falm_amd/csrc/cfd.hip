@@ -430,7 +430,7 @@ __global__ __launch_bounds__(KM_NT) void k_pseudo_u_km(KmTiling kt, Geom g, T Re
 // flux and g along z from the previous plane's registers, g's x and y
 // neighbours and the other fluxes from cache lines of the row.  The arithmetic
 // is k_pseudo_u's, expression by expression.  512 x 128 x 128 in double: 461 ->
-// 340 us (1.54 GB of operands, 4.5 TB/s).
+// 330 us (1.54 GB of operands, 4.7 TB/s).
 template <int SCHEME, class T>
 __global__ __launch_bounds__(KM_NT) void k_pseudo_u_fm(KmTiling kt, Geom g, T ReI, T dt, Vec3<T> un, Vec3<T> u,
                                                        Vec3<T> uu, Vec3W<T> ua, const T *__restrict__ nut,
@@ -1351,10 +1351,9 @@ __global__ __launch_bounds__(K7_NT) void k_sgs_div_km(K7Tiling kt, Geom g, T Cs,
 
 // k_smagorinsky as the step driver's kernel walks it, with the metric fields
 // read instead of the tables (the C-ABI operation on large domains); the
-// expressions are k_smagorinsky's.  512 x 128 x 128 in double: 154 -> 131 us (537 MB, 4.1 TB/s;
-// the square and cube roots take about 30 us of it).  The projection walked
-// the same way measured 309 us against k_project's 291, so it stays a thread
-// per cell.
+// expressions are k_smagorinsky's.  512 x 128 x 128 in double: 154 -> 118 us (537 MB, 4.6 TB/s).
+// The projection walked the same way measured 309 us against k_project's 291,
+// so it stays a thread per cell.
 template <class T>
 __global__ __launch_bounds__(K7_NT) void k_smagorinsky_fm(K7Tiling kt, Geom g, T Cs, Vec3<T> u, T *__restrict__ nut,
                                                           MetField<T> met) {
@@ -1538,16 +1537,12 @@ static falm_status pseudo_u_field_t(const falm_domain *dom, int scheme, double R
     const size_t n = ncell_of(dom);
     KmTiling kt = make_km_tiling(interior_box(g));
     if (kt.blocks == 0) return FALM_OK;
-    // one round: two workgroups a CU in float, one in double (180 VGPRs); 512
-    // x 128 x 128 in double 548 us a predictor with two chunks of 64 planes,
-    // 574 with eight of 16
-    int tk = (sizeof(T) == 4 ? 2 : 1) * 256 / (kt.tx * kt.ty);
-    if (tk < 1) tk = 1;
-    kt.kc = (kt.box.n[2] + tk - 1) / tk;
-    kt.tk = (kt.box.n[2] + kt.kc - 1) / kt.kc;
-    kt.blocks = kt.tx * kt.ty * kt.tk;
     if (!marches(g, n, sizeof(T)))
         return pseudo_u_t<T>(dom, scheme, ReI, dt, un, u, uu, ua, nut, met, ff, nullptr, 23.0, s);
+    // two workgroups a CU in float, one in double (180 VGPRs)
+    kt.kc = k7_chunk_rounds(kt.tx * kt.ty, kt.box.n[2], (sizeof(T) == 4 ? 2 : 1) * cu_count(), 1);
+    kt.tk = (kt.box.n[2] + kt.kc - 1) / kt.kc;
+    kt.blocks = kt.tx * kt.ty * kt.tk;
     TimedLaunch tm(FALM_TIME_PSEUDO_U, s);
 #define FALM_PUF(S)                                                                                              \
     hipLaunchKernelGGL((k_pseudo_u_fm<S, T>), dim3(kt.blocks), dim3(KM_NT), 0, s, kt, g, (T)ReI, (T)dt,          \
@@ -1640,7 +1635,11 @@ static falm_status smag_field_t(const falm_domain *dom, double Cs, const void *u
     const Geom g = make_geom(dom);
     const size_t n = ncell_of(dom);
     if (!marches(g, n, sizeof(T))) return smag_t<T>(dom, Cs, u, nut, met, s);
-    const K7Tiling kt = make_k7_tiling_fit(interior_box(g), 512);  // one round, two a CU (88 VGPRs in double)
+    K7Tiling kt = make_k7_tiling(interior_box(g));
+    // three workgroups a CU in float, two in double (88 VGPRs)
+    kt.kc = k7_chunk_rounds(kt.tx * kt.ty, kt.box.n[2], (sizeof(T) == 4 ? 3 : 2) * cu_count(), 1);
+    kt.tk = (kt.box.n[2] + kt.kc - 1) / kt.kc;
+    kt.blocks = kt.tx * kt.ty * kt.tk;
     TimedLaunch tm(FALM_TIME_SGS, s);
     hipLaunchKernelGGL((k_smagorinsky_fm<T>), dim3(kt.blocks), dim3(K7_NT), 0, s, kt, g, (T)Cs, v3<T>(u, n),
                        (T *)nut, met);

@@ -372,6 +372,9 @@ struct ReduceScratch {
     size_t max_blocks = 0;
 };
 falm_status reduce_scratch(size_t nblocks, ReduceScratch **out);
+
+// compute units of the current device
+int cu_count();
 // device address of falm_dot_noalloc's workspace on the current device,
 // taken on first use (falm_init calls it for its device)
 falm_status noalloc_setup(double **out);

@@ -12,6 +12,8 @@
 // LDS planes are double-buffered: one barrier per plane.
 #pragma once
 
+#include <climits>
+
 #include "common.hpp"
 
 namespace falm {
@@ -65,6 +67,29 @@ inline K7Tiling make_k7_tiling(const Box &b, int max_blocks = RED_BLOCKS) {
     }
     if (b.n[0] <= 0 || b.n[1] <= 0 || b.n[2] <= 0) t.blocks = 0;
     return t;
+}
+
+// Planes per chunk of a kernel on large domains, of which `slots` workgroups
+// are resident at once.  Its time is the rounds of them times a chunk's steps,
+// its planes and `more` of its own; for each number of rounds the shortest
+// chunk that fits them is tried.  A single round of whole chunks (slots / cols
+// of them, rounded down) leaves the chip half empty where the columns are more
+// than half the slots: the pseudo-velocity with per-cell metrics in double, one
+// workgroup a CU, took 497 us at 513 x 128 x 128 (144 columns of 128 planes)
+// and takes 377 (four rounds, seven chunks of 19); 521 -> 373 at 640 x 213 x 61
+// (270 columns); 335 -> 328 at 512 x 128 x 128 (128 columns, one round).
+inline int k7_chunk_rounds(int cols, int nz, int slots, int more) {
+    const long first = ((long)cols + slots - 1) / slots;
+    int kc = nz;
+    long best = LONG_MAX;
+    for (long r = first; r < first + 16; r++) {
+        const long tk = r * slots / cols < nz ? r * slots / cols : nz, k = (nz + tk - 1) / tk;
+        const long cost = r * (k + more);
+        if (cost >= best) continue;
+        best = cost;
+        kc = (int)k;
+    }
+    return kc;
 }
 
 // the shortest chunk whose grid fits max_blocks

@@ -71,6 +71,16 @@ falm_status reduce_scratch(size_t nblocks, ReduceScratch **out) {
     return FALM_OK;
 }
 
+int cu_count() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    return cus;
+}
+
 // --------------------------------------------------------------- timing
 struct TimingState {
     int family = FALM_TIME_NONE;
