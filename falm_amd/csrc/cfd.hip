@@ -1518,14 +1518,25 @@ static falm_status pseudo_u_t(const falm_domain *dom, int scheme, double ReI, do
 }
 
 // Whether a C-ABI operation with per-cell metric fields takes its k-marching
-// form: where a column stays below 4 GiB (32-bit byte offsets) and from 2 M
-// interior cells on.  Below, a thread per cell is as fast or faster (its loads
-// hit the caches, and its grid fills the chip): predictor of 133 x 67 x 45
-// cells in float 23 us against 26, 200 x 100 x 90 in float 59 us both, 256 x 96
-// x 96 in double 180 us against 164, 512 x 128 x 128 652 us against 548.
+// form: from 2 M interior cells on, where a column stays below 4 GiB (32-bit
+// byte offsets).  Below, a thread per cell is as fast or faster (its loads hit
+// the caches, and its grid fills the chip).  In double marching wins from there
+// on over 52 boxes of many shapes (pseudo-velocity 0.61 to 0.93 of the other
+// form's time, Smagorinsky 0.71 to 0.98).  In float the other form keeps up
+// while its planes are small enough for the L2 to hold those that a cell's k
+// neighbours come from and the fields fit the 256 MiB last-level cache, so
+// marching also needs a plane of `plane` cells or a box of `cells`:
+//   pseudo-velocity  26 k, 2.9 M: 0.74 to 1.03 of the other form's time beyond
+//     the lines (218 -> 176 us at 1024 x 128 x 64, worst 33.7 -> 34.7 at 214 x
+//     154 x 62), 0.94 to 1.16 short of both (38.0 and 41.9 us at 186 x 101 x 118)
+//   Smagorinsky      70 k, 7.8 M: 0.70 to 1.04 (58.8 -> 47.1 us at 512 x 128 x
+//     128, worst 15.1 -> 15.7 at 560 x 129 x 31), 0.95 to 1.26 short of both
+//     (31.6 and 34.9 us at 585 x 81 x 127)
 constexpr long long FM_CELLS = 2000000;
-static bool marches(const Geom &g, size_t ncell, size_t elem) {
-    return interior_box(g).size() >= FM_CELLS && ncell * elem < (size_t(1) << 32);
+static bool marches(const Geom &g, size_t ncell, size_t elem, long long plane, long long cells) {
+    const Box b = interior_box(g);
+    const bool large = elem == 8 || (long long)b.n[0] * b.n[1] >= plane || b.size() >= cells;
+    return b.size() >= FM_CELLS && large && ncell * elem < (size_t(1) << 32);
 }
 
 // The C-ABI pseudo-velocity.
@@ -1537,7 +1548,7 @@ static falm_status pseudo_u_field_t(const falm_domain *dom, int scheme, double R
     const size_t n = ncell_of(dom);
     KmTiling kt = make_km_tiling(interior_box(g));
     if (kt.blocks == 0) return FALM_OK;
-    if (!marches(g, n, sizeof(T)))
+    if (!marches(g, n, sizeof(T), 26000, 2900000))
         return pseudo_u_t<T>(dom, scheme, ReI, dt, un, u, uu, ua, nut, met, ff, nullptr, 23.0, s);
     // two workgroups a CU in float, one in double (180 VGPRs)
     kt.kc = k7_chunk_rounds(kt.tx * kt.ty, kt.box.n[2], (sizeof(T) == 4 ? 2 : 1) * cu_count(), 1);
@@ -1634,7 +1645,7 @@ static falm_status smag_field_t(const falm_domain *dom, double Cs, const void *u
                                 hipStream_t s) {
     const Geom g = make_geom(dom);
     const size_t n = ncell_of(dom);
-    if (!marches(g, n, sizeof(T))) return smag_t<T>(dom, Cs, u, nut, met, s);
+    if (!marches(g, n, sizeof(T), 70000, 7800000)) return smag_t<T>(dom, Cs, u, nut, met, s);
     K7Tiling kt = make_k7_tiling(interior_box(g));
     // three workgroups a CU in float, two in double (88 VGPRs)
     kt.kc = k7_chunk_rounds(kt.tx * kt.ty, kt.box.n[2], (sizeof(T) == 4 ? 3 : 2) * cu_count(), 1);

@@ -1,6 +1,8 @@
 """The single operations that take their k-marching form on large domains
-(pseudo-velocity with every scheme, Smagorinsky) against the oracle, just above the size where they do, with a partial tile in x and y, a
-shorter last chunk and a stretched mesh.  The expressions are those of the
+(pseudo-velocity with every scheme, Smagorinsky) against the oracle, just above
+the sizes where they do (2 M cells in double; in float also planes of 70 k
+cells), with a partial tile in x and y, a shorter last chunk and a stretched
+mesh.  The expressions are those of the
 small-domain kernels: the same bars (1e-12 in double, 1e-5 in float; 1e-11
 for the eddy viscosity, whose cube root differs by an ulp or two)."""
 import ctypes as C
@@ -14,12 +16,11 @@ from tests.helpers import Keep, domain, from_dev, interior_mask, rel_err, smooth
 
 pytestmark = pytest.mark.gpu
 
-N = (130, 129, 121)  # 2 029 170 cells: 3 x 17 columns
-
-
-@pytest.fixture(scope="module")
-def F():
-    dom = domain(N)
+# 2 029 170 cells in 3 x 17 columns, planes of 16 770 (in float the small-domain
+# form); 2 074 051 cells in 10 x 15 columns, planes of 71 519
+@pytest.fixture(scope="module", params=[(130, 129, 121), (601, 119, 29)])
+def F(request):
+    dom = domain(request.param)
     rng = np.random.default_rng(8)
     _, (xyz, kx, g, ja) = uniform_metrics(dom, stretch=0.004)
     u = smooth_field(dom, 3, rng, base=0.8, amp=0.5)
