@@ -444,9 +444,14 @@ static hipError_t readback_share(Readback &rb, int w, const T *src, double *out,
     }
 }
 
-// Fields from two chunks on are copied by the threads: at 0.6 M values that is
-// 6 % faster than one pageable copy, and starting the threads costs 0.1 ms.
-static constexpr size_t kReadbackMin = 2 * Readback::kChunk;
+// Fields from four chunks on are copied by the threads, once there are pinned
+// chunks: at 1.1 M values that takes 407 us against one pageable copy's 500 from
+// doubles and 452 against 466 from floats, at 0.8 M 309 against 355 and 340
+// against 311 (starting the threads costs 0.1 ms).  Pinning the chunks takes 1
+// to 2 ms, which a program that takes one snapshot of a case does not get back:
+// a case copies this many values the plain way before it pins them (about what
+// the threads then save), and at once for a field of that size.
+static constexpr size_t kReadbackMin = 4 * Readback::kChunk, kReadbackPay = 8000000;
 
 // Host copy of a field with several threads.  What bounds it is the host: a
 // pageable copy moves 10 GB/s, and on one core the conversion from float and
@@ -561,7 +566,8 @@ falm_status falm_case_get_field(falm_case *C, int field, double *host_out, size_
     FALM_HIP(hipStreamSynchronize(C->stream));
     if (n >= kReadbackMin) {
         std::lock_guard<std::mutex> lk(C->rb.mx);
-        if (C->rb.alloc()) {
+        C->rb.asked += n;
+        if (C->rb.asked >= kReadbackPay && C->rb.alloc()) {
             FALM_HIP(prec == FALM_F64 ? readback(C->rb, (const double *)src, host_out, n, C->stream)
                                       : readback(C->rb, (const float *)src, host_out, n, C->stream));
             return FALM_OK;

@@ -16,6 +16,7 @@ struct Readback {
     static constexpr size_t kChunk = (size_t)1 << 18;  // elements; 2 MiB of doubles
     double *pin = nullptr;                             // 2 kThreads chunks, pinned, kept with the case
     hipEvent_t ev[2 * kThreads] = {};
+    size_t asked = 0;                                  // values of the copies so far
     std::mutex mx;                                     // one call at a time uses the chunks
     bool alloc();
     void release();
