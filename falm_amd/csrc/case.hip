@@ -20,7 +20,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -472,7 +472,7 @@ static hipError_t readback(Readback &rb, const T *src, double *out, size_t n, hi
                 hipError_t ew = hipSetDevice(dev);
                 err[w] = ew == hipSuccess ? readback_share(rb, w, src, out, n, next, s) : ew;
             });
-        } catch (const std::system_error &) {
+        } catch (const std::exception &) {  // no thread, or no memory for one
             break;  // the threads there are share the chunks
         }
     }
