@@ -836,10 +836,10 @@ inline int p2_tiles(int n, int region) {
     return 2 + (rest > 0 ? (rest + o - 1) / o : 0);
 }
 // One double workgroup runs on a CU (164 VGPRs, 115 KB of LDS), so the time is
-// the rounds of 256 workgroups times a chunk's steps; a chunk of n planes takes
+// the rounds of a workgroup a CU times a chunk's steps; a chunk of n planes takes
 // n + 11 (n + 7 at the domain's lower end), of which the first six and the last
 // two do one half-sweep pair of the two.
-inline P2Tiling make_p2_tiling(const Box &b) {
+inline P2Tiling make_p2_tiling(const Box &b, int cus) {
     P2Tiling t;
     t.box = b;
     t.tx = p2_tiles(b.n[0], 64);
@@ -852,7 +852,7 @@ inline P2Tiling make_p2_tiling(const Box &b) {
     for (int kc = 1; kc <= b.n[2]; kc++) {
         const long tk = (b.n[2] + kc - 1) / kc;
         if (tk > 1 && cols * tk > RED_BLOCKS) continue;  // beyond that many columns: whole ones
-        const long cost = ((cols * tk + 255) / 256) * (kc + 7);
+        const long cost = ((cols * tk + cus - 1) / cus) * (kc + 7);
         if (cost >= best) continue;
         best = cost;
         t.kc = kc;
@@ -2691,7 +2691,7 @@ falm_status falm_solver_create(const falm_domain *dom, const falm_solver_config 
         S->tp = make_tiling(pb);
         if (!even || S->tl.tiles == 0) S->tp.tiles = 0;
     }
-    S->p2 = make_p2_tiling(interior_box(S->g));
+    S->p2 = make_p2_tiling(interior_box(S->g), cus);
     S->s2 = make_s2_tiling(interior_box(S->g));
     falm_status st = solver_alloc(S);
     if (st != FALM_OK) {
