@@ -1554,7 +1554,8 @@ __global__ __launch_bounds__(FIN_NT) void k_fin_resnorm(DevState *st, const doub
 // the rest loads, the norms' sums) and 0.7 to 1.1 us an iteration: 10 us at
 // K = 4, 11.2 at 6, 12.2 at 7, and 0.8 at 7 for the division (those figures are
 // with a product by the stored reciprocal and one fused correction, which is not
-// always the rounded quotient and not one at all for infinite or tiny values).
+// always the rounded quotient and not one at all for infinite or tiny values;
+// a second correction and a test for such values take longer than the division).
 // More iterations need a wider ring, so the smallest domains take the most: the
 // line lies where each workgroup sums all partials and every workgroup finds a
 // CU of its own.

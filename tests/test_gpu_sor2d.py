@@ -1,8 +1,8 @@
 """The SOR solver on one interior layer (several iterations a launch, stopped
 in the middle of a launch, at its end and by maxit) against the oracle's
-sweeps: the same iterations, the same x and residual.  Both apply the same
-expression cell by cell; only fused multiply-adds differ, 1e-12 after tens of
-contracting sweeps."""
+sweeps: the same iterations, the same x and residual.  The kernel adds a
+cell's seven products in another order and fused: 1e-12 after tens of
+contracting sweeps.  Its quotients are the rounded ones."""
 import numpy as np
 import pytest
 
@@ -100,3 +100,31 @@ def test_sor_one_layer_infinite_value(gpu, bad, at):
     assert np.isinf(x_ref).any() and not np.isnan(x_ref).any()
     assert np.array_equal(got[~fin], x_ref[~fin])
     assert np.max(np.abs(got[fin] - x_ref[fin])) < 1e-12 * np.max(np.abs(x_ref[fin]))
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_sor_one_layer_quotient(gpu, wide):
+    """The update's quotient is the rounded one, bit for bit: with a diagonal
+    operator, x = 0 and relax 1 one iteration leaves b / ac.  Significands at
+    the ends and in the middle of their range; wide: exponents over the whole
+    range, subnormal numbers and quotients among them."""
+    dom = domain((64, 64, 1))
+    rng, nc, m = np.random.default_rng(11), dom.ncell, interior_mask(dom)
+
+    def numbers(lo, hi):
+        s = rng.integers(0, 1 << 52, nc)
+        k = rng.integers(0, 5, nc)
+        s = np.where(k == 0, s & 15, np.where(k == 1, (1 << 52) - 1 - (s & 15), s))
+        return np.ldexp(1.0 + s / 2.0**52, rng.integers(lo, hi + 1, nc)) * rng.choice((-1.0, 1.0), nc)
+
+    ac, b = numbers(-3, 3), numbers(-3, 3) * m
+    if wide:
+        # (b so that the square of the residual, an ulp of b, is finite)
+        ac, b = numbers(-1040, 1000), numbers(-1040, 500) * m
+        b = np.where(np.abs(np.log2(np.abs(b) + 1e-320) - np.log2(np.abs(ac))) < 1000, b, 0.0)
+    a = np.concatenate([ac, np.zeros(6 * nc)])
+    cfg = abi.solver_config(type=abi.LS_SOR, maxit=5, tol=1e300, relax=1.0, pc_type=abi.LS_EMPTY)
+    dx = to_dev(np.zeros(nc))
+    info = gpu.Solver(dom, cfg).solve(to_dev(a), dx, to_dev(b), None)
+    assert info.it == 1
+    assert np.array_equal(from_dev(dx)[m], (b / ac)[m])
