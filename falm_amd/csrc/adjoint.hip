@@ -441,8 +441,9 @@ __global__ void k_adj_scale_interior(Box ib, Geom g, double dt, F3 ffb) {
 // theirs), while T_dz of the planes above and below stay in registers.  The
 // square root, the cube root and the division are so evaluated 1.4 times a
 // cell (6 times in a thread-per-cell gather), and an output takes one atomic
-// add against the scatter's 18 a cell: 264 -> 79 us at 256 x 96 x 96.  It is
-// bound by the FP64 instructions of a plane.
+// add against the scatter's 18 a cell: 264 -> 79 us at 256 x 96 x 96 called in a
+// row, 263 -> 101 among the other stages.  It is bound by the FP64 instructions
+// of a plane.
 constexpr int AS_X = 64, AS_Y = 8, AS_NT = AS_X * AS_Y;
 __global__ __launch_bounds__(AS_NT) void k_adj_sgs(Box xb, int tx, int ty, int kc, Geom g, double Cs, C3 u, C3 kx,
                                                    const double *__restrict__ ja, const double *__restrict__ nutb,

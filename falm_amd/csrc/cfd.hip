@@ -430,7 +430,7 @@ __global__ __launch_bounds__(KM_NT) void k_pseudo_u_km(KmTiling kt, Geom g, T Re
 // flux and g along z from the previous plane's registers, g's x and y
 // neighbours and the other fluxes from cache lines of the row.  The arithmetic
 // is k_pseudo_u's, expression by expression.  512 x 128 x 128 in double: 461 ->
-// 330 us (1.54 GB of operands, 4.7 TB/s).
+// 340 us (1.54 GB of operands, 4.5 TB/s).
 template <int SCHEME, class T>
 __global__ __launch_bounds__(KM_NT) void k_pseudo_u_fm(KmTiling kt, Geom g, T ReI, T dt, Vec3<T> un, Vec3<T> u,
                                                        Vec3<T> uu, Vec3W<T> ua, const T *__restrict__ nut,
@@ -1351,7 +1351,8 @@ __global__ __launch_bounds__(K7_NT) void k_sgs_div_km(K7Tiling kt, Geom g, T Cs,
 
 // k_smagorinsky as the step driver's kernel walks it, with the metric fields
 // read instead of the tables (the C-ABI operation on large domains); the
-// expressions are k_smagorinsky's.  512 x 128 x 128 in double: 154 -> 118 us (537 MB, 4.6 TB/s).
+// expressions are k_smagorinsky's.  512 x 128 x 128 in double: 154 -> 128 us among a step's other calls
+// (537 MB, 4.2 TB/s), 145 -> 118 called in a row.
 // The projection walked the same way measured 309 us against k_project's 291,
 // so it stays a thread per cell.
 template <class T>
