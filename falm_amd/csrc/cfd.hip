@@ -1522,7 +1522,7 @@ static falm_status pseudo_u_t(const falm_domain *dom, int scheme, double ReI, do
 // form: from 2 M interior cells on, where a column stays below 4 GiB (32-bit
 // byte offsets).  Below, a thread per cell is as fast or faster (its loads hit
 // the caches, and its grid fills the chip).  In double marching wins from there
-// on over 52 boxes of many shapes (pseudo-velocity 0.61 to 0.93 of the other
+// on over 31 boxes of many shapes (pseudo-velocity 0.61 to 0.99 of the other
 // form's time, Smagorinsky 0.71 to 0.98).  In float the other form keeps up
 // while its planes are small enough for the L2 to hold those that a cell's k
 // neighbours come from and the fields fit the 256 MiB last-level cache, so
